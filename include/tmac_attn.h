@@ -346,7 +346,9 @@ int tmac_layer_attention_paged(tmac_context* ctx, tmac_stream stream, int kv_dty
  * in the context's workspace (n_seq * n_kv_head * 16 KiB per 64 rows, rounded
  * up to 256 rows), which grows on demand; a call that needs it to grow while
  * the stream is capturing returns TMAC_ERR_CAPTURE, so run the largest shape
- * once before capture. */
+ * once before capture.  Few queries after many rows: the rows are cut into runs
+ * and a third launch merges their partials, also in the workspace (where that
+ * cannot grow for them, the rows stay whole: the same results up to rounding). */
 int tmac_attention_prefill(tmac_context* ctx, tmac_stream stream, const float* q, const float* k_cache,
                            const float* v_cache, float* out, int n_seq, int n_q, int prefix_len,
                            int64_t seq_stride, int n_head, int n_kv_head, int head_dim);
@@ -379,7 +381,8 @@ int tmac_attention_prefill_paged(tmac_context* ctx, tmac_stream stream, int kv_d
  *   tmac_attention_prefill_tiles: the attention of tmac_attention_prefill over the tiles,
  *     which must hold rows 0 .. prefix_len + n_q - 1 (prefix_len + n_q <= capacity).
  * pack_rows(0, prefix_len + n_q) then attention_prefill_tiles gives the outputs of
- * tmac_attention_prefill bit for bit (the same kernels on the same tiles). */
+ * tmac_attention_prefill bit for bit (the same kernels on the same tiles; under capture,
+ * if the workspace has held the same shape's runs before). */
 size_t tmac_prefill_tiles_bytes(int n_seq, int n_kv_head, int capacity);
 int tmac_prefill_pack_rows(tmac_context* ctx, tmac_stream stream, int kv_dtype, const void* k_cache,
                            const void* v_cache, int64_t seq_stride, void* tiles, int capacity, int n_seq,

@@ -383,3 +383,30 @@ def test_prefill_random_cases(ctx, seed):
     got = run(ctx, q, k, v, n_seq, n_q, prefix, cap, n_head, n_kv)
     ref = oracle.prefill(q, k, v, n_seq, n_q, prefix, cap, n_head, n_kv, HD, n_threads=8)
     assert_close(got, ref, f"seed {seed}: {n_seq}x{n_q} prefix {prefix} cap {cap} heads {n_head}/{n_kv}")
+
+
+@pytest.mark.parametrize("n_seq,n_q,prefix,n_head,n_kv", [
+    (1, 1, 1023, 14, 2),    # one query, every run whole
+    (1, 16, 1016, 14, 2),   # the last run holds keys that only half of the block's queries see
+    (1, 17, 4000, 14, 2),   # a second block with one query
+    (1, 100, 4000, 14, 2),  # 7 blocks of 17 stages, the last with 4 queries
+    (2, 33, 2000, 1, 1), (1, 40, 3000, 8, 1), (1, 31, 5000, 16, 4)])
+def test_prefill_key_runs(ctx, n_seq, n_q, prefix, n_head, n_kv):
+    """Few query blocks after a long prefix: each block's keys are cut into runs of stages
+    (one workgroup each) and merged by a second launch.  Against the oracle on bf16-exact
+    inputs, and the tile-copy entry point bit for bit, into a NaN-filled output."""
+    cap = prefix + n_q
+    q, k, v = (bf16_round(a) for a in make(900 + n_q, n_seq, n_q, prefix, cap, n_head, n_kv))
+    got = run(ctx, q, k, v, n_seq, n_q, prefix, cap, n_head, n_kv)
+    ref = oracle.prefill(q, k, v, n_seq, n_q, prefix, cap, n_head, n_kv, HD, n_threads=8)
+    assert_close(got, ref, f"key runs {n_seq}x{n_q} prefix {prefix} heads {n_head}/{n_kv}")
+    dq, dk, dv = ctx.upload(q), ctx.upload(k), ctx.upload(v)
+    tiles = ctx.empty(ctx.prefill_tiles_bytes(n_seq, n_kv, cap), np.uint8)
+    out = ctx.empty((n_seq, n_q, n_head * HD))
+    out.fill_bytes(0xFF)
+    ctx.prefill_pack_rows(dk, dv, cap, tiles, cap, n_seq, n_kv, HD, 0, cap)
+    ctx.prefill_tiles(dq, tiles, cap, out, n_seq, n_q, prefix, n_head, n_kv, HD)
+    np.testing.assert_array_equal(out.numpy().view(np.uint32), got.view(np.uint32).reshape(out.shape))
+    for d in (dq, dk, dv, tiles, out):
+        d.free()
+    assert ctx.check_device_error() == 0

@@ -111,11 +111,20 @@ struct PrefillArgs {
     int n_pages;
     int* err;                // bit 2: a block-table entry outside the pool (clamped)
     int row_lo;              // pack: first row written
+    // attention: schedule.  Unit = (query block, run of `split` stages of its
+    // keys); split 0: one unit per block.  With more than one unit a block's
+    // partials go to `part` [(sequence, kv head)][block][n_parts][head in the
+    // group][kPrefillPartFloats].
+    int n_sk;                // n_seq * n_kv_head
+    int split;
+    int n_parts;             // units of the last block (the longest), at least 1
+    float* part;
 };
 constexpr int kPrefillQueries = 16;  // queries per workgroup (one MFMA column block)
 constexpr int kPrefillKeys = 64;     // keys per tile
 constexpr int kPrefillTileElems = 2 * 64 * 64;  // bf16 per packed tile: K [key][dim], then V^T [dim][key]
 constexpr int kPrefillStageTiles = 4;           // tiles per LDS stage (two per wave and head pair)
+constexpr int kPrefillPartFloats = 18 * 64;     // one head's partial of a key run: acc [16][64 lanes], m, l
 constexpr int kPrefillWaves = 8;     // waves per workgroup: 4 head pairs x 2 stage halves
 
 struct RopeArgs {

@@ -2000,11 +2000,17 @@ TMAC_DECODE_KERNELS(8, 1)
 // global-to-LDS loads (no registers, no conversion), four tiles per stage,
 // double-buffered, one barrier per stage.
 //
-// Attention workgroup = (16-query block, kv head, sequence), 8 waves.  The
-// 1-D grid is ordered so that the blocks of one (sequence, kv head) run on the
-// same XCD (workgroups are dealt to the 8 XCDs round-robin) and share its L2
-// copy of that head's tiles; within an XCD the longest query blocks start
-// first.  Wave w computes tiles 2 * (w / 4) and 2 * (w / 4) + 1 of every stage
+// Attention workgroup = (16-query block, kv head, sequence), or a run of its
+// keys, 8 waves.  The 1-D grid holds the blocks from the last (most keys) to
+// the first, the (sequence, kv head) pairs of a block side by side: workgroups
+// are dealt to the 8 XCDs round-robin, so every XCD gets an even mix of long
+// and short blocks, longest first, and with 1, 2, 4 or a multiple of 8 pairs
+// an XCD reads only its own share of the tiles.  (An order that gave each XCD
+// a contiguous run of blocks left the XCDs with the last blocks of a prompt
+// working alone: one prompt of 2999 rows 80.5 us, 49.2 in this order.)
+// Where the blocks are fewer than the CUs, each block's keys are cut into runs
+// of `split` stages, one workgroup each, and a second launch merges the
+// partials (prefill_plan in tmac_attn.cpp).  Wave w computes tiles 2 * (w / 4) and 2 * (w / 4) + 1 of every stage
 // for the query heads 2p and 2p + 1 of the group (p = w % 4; a missing second
 // head repeats the first and is not stored), so every K and V^T operand read
 // from LDS feeds two heads' MFMAs.  Each wave works transposed,
@@ -2165,6 +2171,42 @@ __device__ __forceinline__ void prefill_pack_body(const PrefillArgs& a) {
     }
 }
 
+// Stages of keys (kPrefillStageTiles tiles each) that query block b attends.
+__device__ __forceinline__ int prefill_stages(const PrefillArgs& a, int b) {
+    const int kmax = a.prefix_len + min((b + 1) * kPrefillQueries, a.n_q) - 1;
+    return kmax / (kPrefillKeys * kPrefillStageTiles) + 1;
+}
+
+// Unit `rank` of a (sequence, kv head), blocks from the last (most keys) to
+// the first: its query block, which run of `split` stages of the block's keys
+// it attends and how many runs the block has.  Every wave computes the same
+// answer (lane l takes block l of a round of 64; blocks number a few per CU
+// where keys are split).
+__device__ __forceinline__ bool prefill_unit(const PrefillArgs& a, int rank, int& qblk, int& part, int& n_act) {
+    if (a.split == 0) {
+        qblk = a.n_qblk - 1 - rank;
+        return qblk >= 0;
+    }
+    const int lane = threadIdx.x & 63;
+    int base = 0;
+    for (int r0 = 0; r0 < a.n_qblk; r0 += 64) {
+        const int b = a.n_qblk - 1 - r0 - lane;
+        const int u = b >= 0 ? (prefill_stages(a, b) + a.split - 1) / a.split : 0;
+        const int incl = wave_incl_scan(u);
+        const int total = __builtin_amdgcn_readlane(incl, 63);
+        if (rank < base + total) {
+            const unsigned long long hit = __ballot(rank < base + incl);
+            const int first = __builtin_amdgcn_readfirstlane(__ffsll((long long)hit) - 1);
+            qblk = a.n_qblk - 1 - r0 - first;
+            n_act = __builtin_amdgcn_readlane(u, first);
+            part = rank - (base + __builtin_amdgcn_readlane(incl, first) - n_act);
+            return true;
+        }
+        base += total;
+    }
+    return false;
+}
+
 template <int G, int KV>
 __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
     constexpr int NH = KV * G;
@@ -2175,19 +2217,16 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int pair = wave & 3, part = wave >> 2;  // head pair, half of the stage (two tiles)
 
-    // XCD-aware block order: XCD x (= blockIdx.x % 8) owns a contiguous run of
-    // the logical block range.
-    const int n_blk = gridDim.x, xcd = blockIdx.x & 7;
-    const int per = n_blk >> 3, rem = n_blk & 7;
-    const int logical = xcd * per + min(xcd, rem) + (blockIdx.x >> 3);
-    const int sk = logical / a.n_qblk;                  // (sequence, kv head)
-    const int qblk = a.n_qblk - 1 - (logical - sk * a.n_qblk);
+    const int sk = blockIdx.x % a.n_sk;  // (sequence, kv head)
+    int qblk, part_idx = 0, n_act = 1;
+    if (!prefill_unit(a, blockIdx.x / a.n_sk, qblk, part_idx, n_act)) return;
     const int seq = sk / KV, kv = sk - seq * KV;
     const int q0 = qblk * QB;
     const int q_last = min(q0 + QB, a.n_q) - 1;
     const int kmax = a.prefix_len + q_last;  // last key any query of the block attends
     const int n_tiles = kmax / KT + 1;
-    const int n_stages = (n_tiles + NT - 1) / NT;
+    const int st_first = part_idx * a.split;
+    const int n_stages = a.split ? min(st_first + a.split, (n_tiles + NT - 1) / NT) : (n_tiles + NT - 1) / NT;
     const __bf16* slab = reinterpret_cast<const __bf16*>(a.packed) + (size_t)sk * a.n_tp * kPrefillTileElems;
 
     // Two stage buffers as separate objects, so that the compiler sees that a
@@ -2200,7 +2239,9 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
     const bool compute = 2 * pair < G;
     const int hl[2] = {min(2 * pair, G - 1), min(2 * pair + 1, G - 1)};
     const int qi = q0 + col;
-    const int ap = a.prefix_len + qi;  // absolute position of this lane's query
+    // Absolute position of this lane's query.  Columns past the chunk repeat its last query: they must not see
+    // keys past it, whose rows may hold anything (a large score there would raise the wave's running maxima).
+    const int ap = a.prefix_len + min(qi, a.n_q - 1);
     const float c = a.qscale;
 
     // Q^T operands: this lane's query, dims 32j + 8*g4 + (0..7).
@@ -2387,10 +2428,10 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
         __syncthreads();
     };
 
-    dma(0, buf0);
+    dma(st_first, buf0);
     __builtin_amdgcn_s_waitcnt(0x0F70);
     __syncthreads();
-    for (int st = 0; st < n_stages; st += 2) {
+    for (int st = st_first; st < n_stages; st += 2) {
         stage(st, buf0, buf1);
         if (st + 1 < n_stages) stage(st + 1, buf1, buf0);
     }
@@ -2416,16 +2457,29 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
         }
     }
     __syncthreads();
-    if (!compute || part > 0 || qi >= a.n_q) return;
+    if (!compute || part > 0) return;
 #pragma unroll
     for (int hh = 0; hh < 2; ++hh) {
         if (hh == 1 && 2 * pair + 1 >= G) break;
         const float* src = mgp + hh * 18 * 64 + lane;
         const float m1 = src[16 * 64], l1 = src[17 * 64];
-        const float mx = fmaxf(m[hh], m1);  // m[hh] is finite: part 0 holds tile 0, whose key 0 every query sees
-        const float a0 = fast_exp2((m[hh] - mx) * c);
+        // One unit per block: m[hh] is finite (part 0 holds tile 0, whose key 0 every query sees).  A later
+        // run of keys may hold none that an early query of the block sees: weights 0, partial (-inf, 0, 0).
+        const float mx = fmaxf(m[hh], m1);
+        const float a0 = (m[hh] == kNegInf) ? 0.f : fast_exp2((m[hh] - mx) * c);
         const float a1 = (m1 == kNegInf) ? 0.f : fast_exp2((m1 - mx) * c);
-        const float inv = 1.f / (a0 * l[hh] + a1 * l1);
+        const float ls = a0 * l[hh] + a1 * l1;
+        if (n_act > 1) {  // a run's partial, in the accumulators' own layout (256-byte stores)
+            float* pp = a.part + ((((size_t)sk * a.n_qblk + qblk) * a.n_parts + part_idx) * G + hl[hh]) *
+                                     kPrefillPartFloats + lane;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) pp[r * 64] = a0 * o[hh][r / 4][r % 4] + a1 * src[r * 64];
+            pp[16 * 64] = (mx == kNegInf) ? kNegInf : mx * c;
+            pp[17 * 64] = ls;
+            continue;
+        }
+        if (qi >= a.n_q) continue;
+        const float inv = 1.f / ls;
         float* op = a.out + (((size_t)seq * a.n_q + qi) * NH + kv * G + hl[hh]) * kHeadDim + 4 * g4;
 #pragma unroll
         for (int db = 0; db < 4; ++db) {
@@ -2439,10 +2493,66 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
     }
 }
 
+// Merge of a block's key runs (one workgroup per (query block, head, sequence),
+// wave db owning output dims 16 db .. 16 db + 15 in the attention kernel's
+// layout); blocks with one run were written by the attention kernel.  The
+// loads of kMergeRuns runs are in flight together.
+template <int G, int KV>
+__device__ __forceinline__ void prefill_combine_body(const PrefillArgs& a) {
+    constexpr int NH = KV * G, kMergeRuns = 8;
+    const int lane = threadIdx.x & 63, db = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = blockIdx.x % G, rest = blockIdx.x / G;
+    const int qblk = rest % a.n_qblk, sk = rest / a.n_qblk;
+    const int n_act = (prefill_stages(a, qblk) + a.split - 1) / a.split;
+    if (n_act <= 1) return;
+    const float* p0 = a.part + (((size_t)sk * a.n_qblk + qblk) * a.n_parts * G + g) * kPrefillPartFloats + lane;
+    float M = kNegInf, L = 0.f, A[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int u0 = 0; u0 < n_act; u0 += kMergeRuns) {
+        float m[kMergeRuns], l[kMergeRuns], x[kMergeRuns][4];
+#pragma unroll
+        for (int j = 0; j < kMergeRuns; ++j) {
+            const float* p = p0 + (size_t)min(u0 + j, n_act - 1) * G * kPrefillPartFloats;
+            m[j] = p[16 * 64];
+            l[j] = p[17 * 64];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[j][i] = p[(4 * db + i) * 64];
+        }
+        float nm = M;
+#pragma unroll
+        for (int j = 0; j < kMergeRuns; ++j) {
+            m[j] = u0 + j < n_act ? m[j] : kNegInf;
+            nm = fmaxf(nm, m[j]);
+        }
+        // (nm is finite: every column sees key 0, which is in the first run)
+        const float sc = (M == kNegInf) ? 0.f : fast_exp2(M - nm);
+        L *= sc;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) A[i] *= sc;
+#pragma unroll
+        for (int j = 0; j < kMergeRuns; ++j) {
+            const float w = (m[j] == kNegInf) ? 0.f : fast_exp2(m[j] - nm);
+            L = fmaf(l[j], w, L);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) A[i] = fmaf(x[j][i], w, A[i]);
+        }
+        M = nm;
+    }
+    const int qi = qblk * kPrefillQueries + (lane & 15);
+    if (qi >= a.n_q) return;
+    const int seq = sk / KV, kv = sk - seq * KV;
+    const float inv = 1.f / L;
+    *reinterpret_cast<float4*>(a.out + (((size_t)seq * a.n_q + qi) * NH + kv * G + g) * kHeadDim + 16 * db +
+                               4 * (lane >> 4)) = make_float4(A[0] * inv, A[1] * inv, A[2] * inv, A[3] * inv);
+}
+
 #define TMAC_PREFILL_KERNEL(G, KV)                                                                    \
     extern "C" __global__ __launch_bounds__(kPrefillWaves * 64) void tmac_prefill_g##G##_kv##KV(      \
         PrefillArgs a) {                                                                              \
         prefill_body<G, KV>(a);                                                                       \
+    }                                                                                                 \
+    extern "C" __global__ __launch_bounds__(256) void                           \
+        tmac_prefill_combine_g##G##_kv##KV(PrefillArgs a) {                                           \
+        prefill_combine_body<G, KV>(a);                                                               \
     }
 #if TMAC_IN_PART(3)
 TMAC_PREFILL_KERNEL(7, 2)

@@ -121,6 +121,7 @@ struct tmac_context {
     // MFMA decode (bf16, fp16, Q8_0): uniform, ragged, paged, layer, paged layer
     std::map<std::pair<int, int>, hipFunction_t> mdecode[kNarrowTypes][5];
     std::map<std::pair<int, int>, hipFunction_t> prefill;     // chunked prefill, (G, KV)
+    std::map<std::pair<int, int>, hipFunction_t> prefill_combine;  // merge of its key runs
     std::map<int, hipFunction_t> prefill_pack[2][4];          // prefill tile packing: [paged][cache type], by KV
     hipFunction_t any[3] = {};  // any-shape decode kernel by mode (shapes with no compiled kernel)
     hipFunction_t k_rope = nullptr, k_copy = nullptr, k_pos = nullptr, k_qkv = nullptr, k_cvt16 = nullptr,
@@ -842,6 +843,10 @@ int tmac_init(tmac_context** out, int device) {
                 if ((e = get_function(ctx, &f, name)) != hipSuccess)
                     return bail(hip_fail(ctx, e, name));
                 ctx->prefill[{sh[0], sh[1]}] = f;
+                std::snprintf(name, sizeof(name), "tmac_prefill_combine_g%d_kv%d", sh[0], sh[1]);
+                if ((e = get_function(ctx, &f, name)) != hipSuccess)
+                    return bail(hip_fail(ctx, e, name));
+                ctx->prefill_combine[{sh[0], sh[1]}] = f;
                 static const char* const pack_type[4] = {"", "bf16_", "f16_", "q8_"};
                 for (int pg = 0; pg < 2; ++pg)
                     for (int dt = 0; dt < 4; ++dt) {
@@ -1244,6 +1249,57 @@ int tmac_kv_convert(tmac_context* ctx, tmac_stream stream, int kv_dtype, const f
     return launch(ctx, ctx->k_cvt16, (unsigned)((n + 255) / 256), 1, 256, (hipStream_t)stream, &a);
 }
 
+// Schedule of the prefill attention: its units are the query blocks, or, with
+// split > 0, runs of `split` stages (256 keys each) of a block's keys whose
+// partials a second launch merges.  One unit runs per CU, so runs pay only
+// while all of them fit the CUs at once (500 units of 8 stages took 96 us where
+// the 250 whole blocks of 16 took 61): the shortest runs that do are taken if
+// the longest block then loses more stages than the merge launch costs.  One
+// sequence, 100 queries after 4000 rows of a Q8_0 cache: 61.2 us whole, 20.5 in
+// runs; 4 such sequences 63.3 and 32.1.
+struct PrefillPlan {
+    int split;        // stages per unit, 0: one unit per block
+    int n_parts;      // units of the longest block
+    int64_t n_blocks; // units of all (sequence, kv head) pairs
+    size_t floats;    // workspace for the partials
+    int n_qblk;
+};
+
+static PrefillPlan whole_blocks(int n_sk, int n_q) {
+    const int n_qblk = (n_q + kPrefillQueries - 1) / kPrefillQueries;
+    return PrefillPlan{0, 1, (int64_t)n_qblk * n_sk, 0, n_qblk};
+}
+
+static PrefillPlan prefill_plan(const tmac_context* ctx, int n_sk, int group, int n_q, int prefix_len) {
+    // a stage takes about 3.4 us, the merge launch and the partials' stores 7
+    constexpr int kMergeStages = 2;
+    PrefillPlan best = whole_blocks(n_sk, n_q);
+    if (best.n_blocks > ctx->n_cu / 2) return best;
+    auto stages = [&](int b) {
+        return (prefix_len + std::min((b + 1) * kPrefillQueries, n_q) - 1) / (kPrefillKeys * kPrefillStageTiles) + 1;
+    };
+    const int n_qblk = best.n_qblk, longest = stages(n_qblk - 1);
+    for (int split = 1; split + kMergeStages < longest; split++) {
+        int64_t units = 0;
+        for (int b = 0; b < n_qblk; b++) units += (stages(b) + split - 1) / split;
+        units *= n_sk;
+        if (units > ctx->n_cu) continue;
+        const int n_parts = (longest + split - 1) / split;
+        return PrefillPlan{split, n_parts, units, (size_t)n_sk * n_qblk * n_parts * group * tmac::kPrefillPartFloats,
+                           n_qblk};
+    }
+    return best;
+}
+
+static int launch_prefill(tmac_context* ctx, hipStream_t stream, int n_head, int n_kv_head, const PrefillPlan& plan,
+                   PrefillArgs& a) {
+    const std::pair<int, int> key{n_head / n_kv_head, n_kv_head};
+    int rc = launch(ctx, ctx->prefill.at(key), (unsigned)plan.n_blocks, 1, kPrefillWaves * 64, stream, &a);
+    if (rc || !plan.split) return rc;
+    return launch(ctx, ctx->prefill_combine.at(key), (unsigned)((int64_t)a.n_sk * a.n_qblk * key.first), 1, 256, stream,
+                  &a);
+}
+
 // Chunked prefill over a contiguous cache (block_table null: sequence s at row
 // s * seq_stride) or a paged one (n_pages pages, block_table [n_seq][max_pages]).
 static int prefill_impl(tmac_context* ctx, tmac_stream stream, int dt, const float* q, const void* k_cache,
@@ -1269,27 +1325,32 @@ static int prefill_impl(tmac_context* ctx, tmac_stream stream, int dt, const flo
     if ((int64_t)((n_q + kPrefillQueries - 1) / kPrefillQueries) * n_kv_head * n_seq > INT_MAX)
         return fail(ctx, TMAC_ERR_INVALID_ARG, "prefill: too many (query block, kv head, sequence) units");
     if (n_seq == 0 || n_q == 0) return TMAC_OK;
-    auto it = ctx->prefill.find({n_head / n_kv_head, n_kv_head});
-    if (it == ctx->prefill.end()) return fail(ctx, TMAC_ERR_UNSUPPORTED, "prefill: unsupported group");
+    if (!ctx->prefill.count({n_head / n_kv_head, n_kv_head}))
+        return fail(ctx, TMAC_ERR_UNSUPPORTED, "prefill: unsupported group");
     if ((rc = set_device(ctx))) return rc;
     // bf16 tiles of rows 0 .. prefix_len + n_q - 1 per (sequence, kv head), in
     // the split-KV workspace, then the attention over them.
-    const int n_qblk = (n_q + kPrefillQueries - 1) / kPrefillQueries;
     const int n_rows = prefix_len + n_q;
     const int n_tp = ((n_rows + kPrefillKeys - 1) / kPrefillKeys + kPrefillStageTiles - 1) / kPrefillStageTiles *
                      kPrefillStageTiles;
     const int64_t pack_blocks = (int64_t)n_tp * n_kv_head * n_seq;
     if (pack_blocks > INT_MAX) return fail(ctx, TMAC_ERR_INVALID_ARG, "prefill: too many cache tiles");
-    const size_t pack_bytes = (size_t)pack_blocks * kPrefillTileElems * sizeof(uint16_t);
-    if ((rc = ensure_workspace(ctx, (hipStream_t)stream, pack_bytes / sizeof(float)))) return rc;
+    const size_t pack_floats = (size_t)pack_blocks * kPrefillTileElems * sizeof(uint16_t) / sizeof(float);
+    PrefillPlan plan = prefill_plan(ctx, n_seq * n_kv_head, n_head / n_kv_head, n_q, prefix_len);
+    rc = ensure_workspace(ctx, (hipStream_t)stream, pack_floats + plan.floats);
+    if (rc && plan.split) {  // no room for the partials (a capturing stream): one unit per block
+        plan = whole_blocks(n_seq * n_kv_head, n_q);
+        rc = ensure_workspace(ctx, (hipStream_t)stream, pack_floats);
+    }
+    if (rc) return rc;
     PrefillArgs a{q, static_cast<const float*>(k_cache), static_cast<const float*>(v_cache), out, seq_stride, n_q,
-                  prefix_len, n_qblk, kQScale, reinterpret_cast<uint16_t*>(workspace(ctx)), n_tp, n_rows, 0, n_tp,
-                  block_table, max_pages, n_pages, ctx->err, 0};
+                  prefix_len, plan.n_qblk, kQScale, reinterpret_cast<uint16_t*>(workspace(ctx)), n_tp, n_rows, 0,
+                  n_tp, block_table, max_pages, n_pages, ctx->err, 0, n_seq * n_kv_head, plan.split, plan.n_parts,
+                  workspace(ctx) + pack_floats};
     if ((rc = launch(ctx, ctx->prefill_pack[block_table ? 1 : 0][dt].at(n_kv_head), (unsigned)pack_blocks, 1, 256,
                      (hipStream_t)stream, &a)))
         return rc;
-    return launch(ctx, it->second, (unsigned)((int64_t)n_qblk * n_kv_head * n_seq), 1, kPrefillWaves * 64,
-                  (hipStream_t)stream, &a);
+    return launch_prefill(ctx, (hipStream_t)stream, n_head, n_kv_head, plan, a);
 }
 
 int tmac_attention_prefill(tmac_context* ctx, tmac_stream stream, const float* q, const float* k_cache,
@@ -1360,7 +1421,7 @@ int tmac_prefill_pack_rows(tmac_context* ctx, tmac_stream stream, int kv_dtype, 
     // other rows of those tiles keep their contents.
     PrefillArgs a{nullptr, static_cast<const float*>(k_cache), static_cast<const float*>(v_cache), nullptr,
                   seq_stride, 0, 0, 0, kQScale, static_cast<uint16_t*>(tiles), n_tp, row_end, t0, t1 - t0,
-                  nullptr, 0, 0, ctx->err, row_begin};
+                  nullptr, 0, 0, ctx->err, row_begin, 0, 0, 1, nullptr};
     return launch(ctx, ctx->prefill_pack[0][dt].at(n_kv_head), (unsigned)blocks, 1, 256, (hipStream_t)stream, &a);
 }
 
@@ -1380,15 +1441,17 @@ int tmac_attention_prefill_tiles(tmac_context* ctx, tmac_stream stream, const fl
     if ((int64_t)((n_q + kPrefillQueries - 1) / kPrefillQueries) * n_kv_head * n_seq > INT_MAX)
         return fail(ctx, TMAC_ERR_INVALID_ARG, "prefill_tiles: too many (query block, kv head, sequence) units");
     if (n_seq == 0 || n_q == 0) return TMAC_OK;
-    auto it = ctx->prefill.find({n_head / n_kv_head, n_kv_head});
-    if (it == ctx->prefill.end()) return fail(ctx, TMAC_ERR_UNSUPPORTED, "prefill_tiles: unsupported group");
+    if (!ctx->prefill.count({n_head / n_kv_head, n_kv_head}))
+        return fail(ctx, TMAC_ERR_UNSUPPORTED, "prefill_tiles: unsupported group");
     if ((rc = set_device(ctx))) return rc;
-    const int n_qblk = (n_q + kPrefillQueries - 1) / kPrefillQueries;
-    PrefillArgs a{q, nullptr, nullptr, out, 0, n_q, prefix_len, n_qblk, kQScale,
+    PrefillPlan plan = prefill_plan(ctx, n_seq * n_kv_head, n_head / n_kv_head, n_q, prefix_len);
+    if (plan.split && ensure_workspace(ctx, (hipStream_t)stream, plan.floats) != TMAC_OK)
+        plan = whole_blocks(n_seq * n_kv_head, n_q);  // no room for the partials: one unit per block, no workspace
+    PrefillArgs a{q, nullptr, nullptr, out, 0, n_q, prefix_len, plan.n_qblk, kQScale,
                   static_cast<uint16_t*>(const_cast<void*>(tiles)), prefill_tiles_per_head(capacity),
-                  prefix_len + n_q, 0, 0, nullptr, 0, 0, ctx->err, 0};
-    return launch(ctx, it->second, (unsigned)((int64_t)n_qblk * n_kv_head * n_seq), 1, kPrefillWaves * 64,
-                  (hipStream_t)stream, &a);
+                  prefix_len + n_q, 0, 0, nullptr, 0, 0, ctx->err, 0, n_seq * n_kv_head, plan.split, plan.n_parts,
+                  workspace(ctx)};
+    return launch_prefill(ctx, (hipStream_t)stream, n_head, n_kv_head, plan, a);
 }
 
 int tmac_pos_update(tmac_context* ctx, tmac_stream stream, int* pos_dev, int value, int add) {
