@@ -40,7 +40,8 @@
  *    entry points tmac_attention_op, tmac_attention_decode_batched /
  *    _ragged / _ragged_noalloc and tmac_layer_attention[_devpos] take any
  *    other n_head a multiple of n_kv_head and any even head_dim up to 256
- *    (one workgroup per query head; scores scaled by 1/sqrt(head_dim)), and
+ *    (scores scaled by 1/sqrt(head_dim); head_dim a multiple of 4 shares each
+ *    row among the group's query heads and splits long rows over workgroups), and
  *    tmac_rope_op / tmac_rope_rows any even head_dim up to 256 (kernel_rope.metal:5-22).
  *    The reference's kernel_attn is one 32-lane simdgroup with 2 dims per lane
  *    (kernel_attn.metal:20-21), so it defines head_dim <= 64 only; above 64 this

@@ -179,3 +179,55 @@ def test_other_entry_points_refuse_other_shapes(ctx):
     assert lib.tmac_attention_decode_paged(h, None, tmac_attn.TMAC_KV_F32, p, p, p, 1, p, 1, p, p, 1, 3, 1, 64, 16,
                                            0) == U
     d.free()
+
+
+@pytest.mark.parametrize("nh,nkv,hd", [(14, 2, 128), (12, 4, 96), (8, 8, 80), (5, 5, 256), (14, 2, 32), (20, 2, 64),
+                                       (3, 1, 64), (2, 2, 4), (9, 3, 12), (9, 3, 66)])
+@pytest.mark.parametrize("n_seq,max_len", [(1, 127), (1, 700), (3, 2050), (40, 300)])
+def test_any_shape_splits(ctx, nh, nkv, hd, n_seq, max_len):
+    """Batched, ragged and layer-step decode of shapes without compiled kernels, at lengths on and
+    around the split, step and wave boundaries (splits are multiples of 32 rows from 128 rows on;
+    heads 20 / 2 take two head tiles).  head_dim 66 keeps the unsplit row kernel."""
+    k = oracle.normal(8000 + hd, (n_seq * max_len, nkv * hd))
+    v = oracle.normal(8001 + hd, (n_seq * max_len, nkv * hd))
+    q = oracle.normal(8002 + nh, (n_seq, nh * hd))
+    offs = np.arange(n_seq, dtype=np.int64) * max_len
+    lens = np.resize(np.array([max_len, 1, 0, 33, 128, 129, 255, 257, max_len - 1], np.int32), n_seq)
+    lens = np.minimum(lens, max_len)
+    dq, dk, dv, do, dl = (ctx.upload(x) for x in (q, k, v, offs, lens))
+    dout = ctx.empty((n_seq, nh * hd))
+    full = oracle.attention_ragged(q, k, v, offs, np.full(n_seq, max_len, np.int32), nh, nkv, hd, n_threads=8)
+    dout.fill_bytes(0xFF)
+    ctx.decode_batched(dq, dk, dv, dout, n_seq, nh, nkv, hd, max_len, max_len)
+    assert_close(dout.numpy(), full, f"batched {nh}/{nkv}/{hd} {n_seq}x{max_len}")
+    nz = lens > 0
+    ref = np.zeros((n_seq, nh * hd), np.float32)
+    ref[nz] = oracle.attention_ragged(q[nz], k, v, offs[nz], lens[nz], nh, nkv, hd, n_threads=8)
+    for call in (ctx.decode_ragged, None):
+        dout.fill_bytes(0xFF)
+        if call:
+            call(dq, dk, dv, do, dl, dout, n_seq, nh, nkv, hd, max_len)
+        else:  # the partials in the fixed scratch array
+            rc = ctx.lib.tmac_attention_decode_ragged_noalloc(ctx.handle, None, dq.ptr, dk.ptr, dv.ptr, do.ptr, dl.ptr,
+                                                              dout.ptr, n_seq, nh, nkv, hd, max_len, 0)
+            assert rc == tmac_attn.TMAC_OK
+        assert_close(dout.numpy(), ref, f"ragged {nh}/{nkv}/{hd} {n_seq}x{max_len}")
+    pos_dev = ctx.upload(np.zeros(1, np.int32))
+    kn, vn = oracle.normal(8003, nkv * hd), oracle.normal(8004, nkv * hd)
+    dkn, dvn = ctx.upload(kn), ctx.upload(vn)
+    ctx.rope_prepare(hd, 1e6, max_len)
+    kc, vc = k[:max_len].copy(), v[:max_len].copy()
+    dkc, dvc = ctx.upload(kc), ctx.upload(vc)
+    for pos in sorted({0, 31, 126, max_len // 2, max_len - 1}):
+        ref1, _, _ = oracle.layer_step(q[0], kn, vn, kc, vc, nh, nkv, hd, pos, 1e6)
+        if pos % 2:
+            ctx.layer_attention(dq, dkn, dvn, dkc, dvc, dout, nh, nkv, hd, pos, max_len, 1e6)
+        else:
+            pos_dev.copy_from(np.array([pos], np.int32))
+            ctx.layer_attention_devpos(dq, dkn, dvn, dkc, dvc, dout, nh, nkv, hd, pos_dev, max_len, 1e6)
+        assert_close(dout.numpy()[0], ref1, f"layer {nh}/{nkv}/{hd} pos {pos} of {max_len}")
+    np.testing.assert_array_equal(dkc.numpy(), kc)
+    np.testing.assert_array_equal(dvc.numpy(), vc)
+    for d in (dq, dk, dv, do, dl, dout, pos_dev, dkn, dvn, dkc, dvc):
+        d.free()
+    assert ctx.check_device_error() == 0

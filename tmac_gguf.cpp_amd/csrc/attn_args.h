@@ -24,6 +24,8 @@ constexpr int kHvWaves = 8;         // split-V head kernel (short contexts): 512
 constexpr int kHvDepth = 2;         // split-V head kernel: steps of K/V in flight per wave
 constexpr int kHvSplitDefault = 8;  // workgroups per query head, each accumulating 64/8 dims of V
 constexpr int kAnyWavesHost = 8;    // any-shape decode kernel (shapes with no compiled kernel): 512 threads
+// any-shape group kernel (head_dim a multiple of 4) with GT query heads per workgroup: waves per workgroup
+constexpr int any_group_waves(int gt) { return gt == 1 ? 8 : 4; }
 constexpr int kAnyMaxDim = 256;     // any-shape kernel and RoPE: even head_dim up to this
 constexpr int kMaxSplits = 256;     // split-KV workgroups per sequence, at most
 constexpr int kPartialStride = kHeadDim + 2;  // per (split, head): acc[64], m, l

@@ -1748,6 +1748,10 @@ __device__ __forceinline__ void combine_sk_body(const DecodeArgs& a) {
 // mode: q and k_new rotated at pos (RoPE pairs (d, d+1) sit in adjacent
 // lanes), the group's first head stores row pos, wave 0 attends it.
 constexpr int kAnyWaves = kAnyWavesHost;
+template <bool V>
+struct BoolTag {
+    static constexpr bool value = V;
+};
 constexpr int kAnyDpl = kAnyMaxDim / 32;  // dims per lane at most
 
 __device__ __forceinline__ float half_sum(float x) {  // sum over the 32 lanes of a half wave
@@ -1925,10 +1929,325 @@ __device__ __forceinline__ void any_body(const DecodeArgs& a) {
     }
 }
 
+// Any-shape decode with GQA sharing (head_dim a multiple of 4; fp32 caches).
+// HBM-bound: the row kernel above reads a kv head's rows once per query head,
+// 4 bytes a lane (14 / 2 heads of 128 dims, 32 x 2048 rows: 142 us, 0.95 TB/s);
+// here a workgroup serves GT query heads of one kv head from one read of the
+// rows (32.6 us, 4.1 TB/s; one sequence of 4096 rows 147 -> 10.4 us).
+// grid = (split, kv head x head tile, sequence), NW waves.  Like the compiled
+// group kernel with runtime head_dim: a row is served by LPR lanes of 8 dims
+// (16-byte chunks c and c + LPR of the head), a wave step covers 64 / LPR rows,
+// kAnyDepth steps of K and V are in flight, the online softmax keeps one
+// running max per (wave, head), raised lazily, and the splits' partials
+// ([sequence][split][head][head_dim + 2]: acc, m, l) are merged by a second
+// launch.  Lanes whose chunk lies past head_dim load chunk 0 and score 0.
+constexpr int kAnyDepth = 3;
+
+template <int L>
+__device__ __forceinline__ float lanes_sum(float x) {  // over L consecutive lanes
+    x += dpp<0xB1>(x);
+    x += dpp<0x4E>(x);
+    if constexpr (L >= 8) x += dpp<0x141>(x);
+    if constexpr (L >= 16) x += dpp<0x140>(x);
+    if constexpr (L >= 32) {
+        const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+        x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    }
+    return x;
+}
+template <int L>
+__device__ __forceinline__ float rows_sum(float x) {  // over the lanes that differ by multiples of L
+    if constexpr (L == 4) {
+        x += dpp<0x128>(x);  // row_ror:8
+        x += dpp<0x124>(x);  // row_ror:4
+        return xor_sum<16>(x);
+    } else {
+        return xor_sum<L>(x);
+    }
+}
+
+template <int LPR, int GT, int NW, int MODE>
+__device__ __forceinline__ void anyg_body(const DecodeArgs& a) {
+    static_assert(MODE == kUniform || MODE == kRagged || MODE == kLayer, "any-shape kernel modes");
+    constexpr int RPS = 64 / LPR;  // rows per wave step
+    const int hd = a.head_dim, n_kv = a.n_kv_head, group = a.n_head / n_kv;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = lane % LPR, slot = lane / LPR;
+    const int split = blockIdx.x, kvh = blockIdx.y % n_kv, g0 = (blockIdx.y / n_kv) * GT, seq = blockIdx.z;
+    const int head0 = kvh * group + g0, n_g = min(GT, group - g0);  // this workgroup's query heads
+    const size_t rowf = (size_t)n_kv * hd;
+    int n_pos, pos;
+    size_t base;
+    if (!seq_geometry<MODE>(a, seq, n_pos, pos, base)) {
+        if (split == 0 && kvh == 0 && g0 == 0 && threadIdx.x == 0) atomicOr(a.err, 1);
+        return;
+    }
+    n_pos = __builtin_amdgcn_readfirstlane(n_pos);
+    pos = __builtin_amdgcn_readfirstlane(pos);
+    float* out = a.out + ((size_t)seq * a.n_head + head0) * hd;
+    const int n_act = (n_pos + a.split_len - 1) / a.split_len;
+    if (n_pos <= 0 || n_act > a.n_splits) {  // no rows: zeros; longer than the max_len the launch was sized for: NaN
+        if (split == 0) {
+            for (int i = threadIdx.x; i < n_g * hd; i += NW * 64) out[i] = n_pos <= 0 ? 0.f : __builtin_nanf("");
+            if (n_pos > 0 && threadIdx.x == 0) atomicOr(a.err, 2);
+        }
+        return;
+    }
+    if (split >= n_act) return;
+    const int mem_rows = MODE == kLayer ? pos : n_pos;  // layer mode: row pos comes from registers
+    const int r0 = split * a.split_len;
+    const int n_rows = max(min(r0 + a.split_len, mem_rows) - r0, 0);
+
+    const bool has0 = 4 * c < hd, has1 = 4 * (c + LPR) < hd;
+    const int d0 = has0 ? 4 * c : 0, d1 = has1 ? 4 * (c + LPR) : 0;  // this lane's dims of a head: d0.., d1..
+    auto load_lane = [&](float (&x)[8], const float* p) {            // fp32 rows of q, k_new, v_new
+        const float4 u = *reinterpret_cast<const float4*>(p + d0), v = *reinterpret_cast<const float4*>(p + d1);
+        x[0] = u.x; x[1] = u.y; x[2] = u.z; x[3] = u.w;
+        x[4] = v.x; x[5] = v.y; x[6] = v.z; x[7] = v.w;
+    };
+    const float2* cs_row = MODE == kLayer ? a.rope_cs + (size_t)pos * (hd / 2) : nullptr;
+    auto rope = [&](float (&x)[8]) {
+        const float4 t0 = *reinterpret_cast<const float4*>(cs_row + d0 / 2);
+        const float4 t1 = *reinterpret_cast<const float4*>(cs_row + d1 / 2);
+        rope8p(x, t0, t1);
+    };
+    const float qscale = 1.4426950408889634f / sqrtf((float)hd);  // log2(e) / sqrt(head_dim)
+    float q[GT][8];
+#pragma unroll
+    for (int g = 0; g < GT; ++g) {
+        load_lane(q[g], a.q + ((size_t)seq * a.n_head + head0 + min(g, n_g - 1)) * hd);
+        if (MODE == kLayer) rope(q[g]);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) q[g][t] *= qscale;
+    }
+    float m[GT], l[GT], acc[GT][8];
+#pragma unroll
+    for (int g = 0; g < GT; ++g) {
+        m[g] = kNegInf;
+        l[g] = 0.f;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) acc[g][t] = 0.f;
+    }
+    auto attend_row = [&](float (&kf)[8], const float (&vf)[8], bool valid, auto masked) {
+        constexpr bool MASKED = decltype(masked)::value;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {  // (chunks past head_dim hold chunk 0 again)
+            kf[t] = has0 ? kf[t] : 0.f;
+            kf[4 + t] = has1 ? kf[4 + t] : 0.f;
+        }
+        float s[GT];
+#pragma unroll
+        for (int g = 0; g < GT; ++g) {
+            float x = q[g][0] * kf[0];
+#pragma unroll
+            for (int t = 1; t < 8; ++t) x = fmaf(q[g][t], kf[t], x);
+            s[g] = lanes_sum<LPR>(x);
+            if (MASKED) s[g] = valid ? s[g] : kNegInf;
+        }
+        float over = s[0] - m[0];
+#pragma unroll
+        for (int g = 1; g < GT; ++g) over = fmaxf(over, s[g] - m[g]);
+        if (__any(over > kTau)) {
+#pragma unroll
+            for (int g = 0; g < GT; ++g) {
+                const float mn = fmaxf(m[g], xor_max<1>(s[g]));
+                const float alpha = (m[g] == kNegInf) ? 0.f : fast_exp2(m[g] - mn);
+                l[g] *= alpha;
+#pragma unroll
+                for (int t = 0; t < 8; ++t) acc[g][t] *= alpha;
+                m[g] = mn;
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < GT; ++g) {
+            const float e = fast_exp2(s[g] - m[g]);
+            l[g] += e;
+#pragma unroll
+            for (int t = 0; t < 8; ++t) acc[g][t] = fmaf(e, vf[t], acc[g][t]);
+        }
+    };
+
+    const float* kb = a.k + (base + r0) * rowf + (size_t)kvh * hd;
+    const float* vb = a.v + (base + r0) * rowf + (size_t)kvh * hd;
+    struct Row {
+        float x[8];
+    };
+    auto load_row8 = [&](Row& r, const float* head_row) {
+        typedef float f32x4_t __attribute__((ext_vector_type(4)));
+        constexpr bool NT = GT > 1;  // one head per workgroup: other workgroups of the kv head read the row too
+        const f32x4_t u = ld<NT, f32x4_t>(reinterpret_cast<const char*>(head_row + d0));
+        const f32x4_t v = ld<NT, f32x4_t>(reinterpret_cast<const char*>(head_row + d1));
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            r.x[t] = u[t];
+            r.x[4 + t] = v[t];
+        }
+    };
+    // Wave w takes full steps w, w + NW, ...; prefetches past the last one are clamped to it (the same order and
+    // scheduling barriers as attend_rows).
+    const int full = n_rows / RPS, nk = (full - wave + NW - 1) / NW;
+    if (nk > 0) {
+        Row kbuf[kAnyDepth], vbuf[kAnyDepth];
+        auto row_at = [&](int k) { return (size_t)((wave + NW * min(k, nk - 1)) * RPS + slot) * rowf; };
+#pragma unroll
+        for (int d = 0; d < kAnyDepth; ++d) {
+            load_row8(kbuf[d], kb + row_at(d));
+            load_row8(vbuf[d], vb + row_at(d));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        for (int k0 = 0; k0 < nk; k0 += kAnyDepth) {
+#pragma unroll
+            for (int d = 0; d < kAnyDepth; ++d) {
+                if (k0 + d < nk) attend_row(kbuf[d].x, vbuf[d].x, true, BoolTag<false>{});
+                load_row8(kbuf[d], kb + row_at(k0 + d + kAnyDepth));
+                load_row8(vbuf[d], vb + row_at(k0 + d + kAnyDepth));
+            }
+        }
+    }
+    if (full * RPS < n_rows && full % NW == wave) {  // the partial last step
+        const int row = full * RPS + slot;
+        Row kr, vr;
+        load_row8(kr, kb + (size_t)min(row, n_rows - 1) * rowf);
+        load_row8(vr, vb + (size_t)min(row, n_rows - 1) * rowf);
+        attend_row(kr.x, vr.x, row < n_rows, BoolTag<true>{});
+    }
+    if (MODE == kLayer && split == n_act - 1 && wave == 0) {
+        // The new token (row pos) by the wave's first row slot: RoPE its k, the group's first tile writes the cache
+        // row (tmac_gguf.cpp:1090-1091), attended from registers.
+        float kn[8], vn[8];
+        load_lane(kn, a.k_new + (size_t)kvh * hd);
+        load_lane(vn, a.v_new + (size_t)kvh * hd);
+        rope(kn);
+        if (slot == 0 && g0 == 0) {
+            float* ko = a.k_out + (size_t)pos * rowf + (size_t)kvh * hd;
+            float* vo = a.v_out + (size_t)pos * rowf + (size_t)kvh * hd;
+            if (has0) {
+                *reinterpret_cast<float4*>(ko + d0) = make_float4(kn[0], kn[1], kn[2], kn[3]);
+                *reinterpret_cast<float4*>(vo + d0) = make_float4(vn[0], vn[1], vn[2], vn[3]);
+            }
+            if (has1) {
+                *reinterpret_cast<float4*>(ko + d1) = make_float4(kn[4], kn[5], kn[6], kn[7]);
+                *reinterpret_cast<float4*>(vo + d1) = make_float4(vn[4], vn[5], vn[6], vn[7]);
+            }
+        }
+        attend_row(kn, vn, slot == 0, BoolTag<true>{});
+    }
+    // row slots -> wave (same max), waves -> LDS
+    __shared__ float s_acc[NW][GT][8 * LPR];
+    __shared__ float s_m[NW][GT], s_l[NW][GT];
+#pragma unroll
+    for (int g = 0; g < GT; ++g) {
+        l[g] = rows_sum<LPR>(l[g]);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) acc[g][t] = rows_sum<LPR>(acc[g][t]);
+        if (slot == 0) {
+            *reinterpret_cast<float4*>(&s_acc[wave][g][4 * c]) = make_float4(acc[g][0], acc[g][1], acc[g][2], acc[g][3]);
+            *reinterpret_cast<float4*>(&s_acc[wave][g][4 * (c + LPR)]) =
+                make_float4(acc[g][4], acc[g][5], acc[g][6], acc[g][7]);
+            if (c == 0) {
+                s_m[wave][g] = m[g];
+                s_l[wave][g] = l[g];
+            }
+        }
+    }
+    __syncthreads();
+    float* ws = n_act > 1 ? a.ws + (((size_t)seq * a.n_splits + split) * a.n_head + head0) * (size_t)(hd + 2) : nullptr;
+    for (int i = threadIdx.x; i < n_g * 8 * LPR; i += NW * 64) {
+        const int g = i / (8 * LPR), d = i % (8 * LPR);
+        if (d >= hd) continue;
+        float M = kNegInf;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) M = fmaxf(M, s_m[w][g]);
+        float L = 0.f, A = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            const float mw = s_m[w][g];
+            const float sc = (mw == kNegInf) ? 0.f : fast_exp2(mw - M);
+            L = fmaf(s_l[w][g], sc, L);
+            A = fmaf(s_acc[w][g][d], sc, A);
+        }
+        if (n_act == 1) {
+            out[(size_t)g * hd + d] = A / L;
+        } else {
+            float* p = ws + (size_t)g * (hd + 2);
+            p[d] = A;
+            if (d == 0) {
+                p[hd] = M;
+                p[hd + 1] = L;
+            }
+        }
+    }
+}
+
+// Merge of the splits: one workgroup per (query head, sequence), thread d
+// owning output dim d; the loads of kAnyMerge splits are in flight together.
+constexpr int kAnyMerge = 8;
+template <int MODE>
+__device__ __forceinline__ void any_combine_body(const DecodeArgs& a) {
+    const int h = blockIdx.x, seq = blockIdx.y, hd = a.head_dim, d = min((int)threadIdx.x, hd - 1);
+    int n_pos, pos;
+    size_t base;
+    if (!seq_geometry<MODE>(a, seq, n_pos, pos, base) || n_pos <= 0) return;
+    const int n_act = (n_pos + a.split_len - 1) / a.split_len;
+    if (n_act <= 1 || n_act > a.n_splits) return;
+    const size_t SP = (size_t)a.n_head * (hd + 2);  // floats between splits
+    const float* ws = a.ws + (size_t)seq * a.n_splits * SP + (size_t)h * (hd + 2);
+    float M = kNegInf, L = 0.f, A = 0.f;
+    for (int u0 = 0; u0 < n_act; u0 += kAnyMerge) {
+        float m[kAnyMerge], l[kAnyMerge], x[kAnyMerge];
+#pragma unroll
+        for (int j = 0; j < kAnyMerge; ++j) {
+            const float* p = ws + (size_t)min(u0 + j, n_act - 1) * SP;
+            m[j] = p[hd];
+            l[j] = p[hd + 1];
+            x[j] = p[d];
+        }
+        float nm = M;
+#pragma unroll
+        for (int j = 0; j < kAnyMerge; ++j) {
+            m[j] = u0 + j < n_act ? m[j] : kNegInf;
+            nm = fmaxf(nm, m[j]);  // finite: every split holds a row
+        }
+        const float sc = (M == kNegInf) ? 0.f : fast_exp2(M - nm);
+        L *= sc;
+        A *= sc;
+#pragma unroll
+        for (int j = 0; j < kAnyMerge; ++j) {
+            const float e = (m[j] == kNegInf) ? 0.f : fast_exp2(m[j] - nm);
+            L = fmaf(l[j], e, L);
+            A = fmaf(x[j], e, A);
+        }
+        M = nm;
+    }
+    if ((int)threadIdx.x < hd) a.out[((size_t)seq * a.n_head + h) * hd + d] = A / L;
+}
+
 #if TMAC_IN_PART(0)
 extern "C" __global__ __launch_bounds__(kAnyWaves * 64) void tmac_decode_u_any(DecodeArgs a) { any_body<kUniform>(a); }
 extern "C" __global__ __launch_bounds__(kAnyWaves * 64) void tmac_decode_r_any(DecodeArgs a) { any_body<kRagged>(a); }
 extern "C" __global__ __launch_bounds__(kAnyWaves * 64) void tmac_layer_any(DecodeArgs a) { any_body<kLayer>(a); }
+#define TMAC_ANYG_KERNEL(M, MODE, LPR, GT)                                                                      \
+    extern "C" __global__ __launch_bounds__(any_group_waves(GT) * 64) void tmac_##M##_any_l##LPR##_g##GT(       \
+        DecodeArgs a) {                                                                                        \
+        anyg_body<LPR, GT, any_group_waves(GT), MODE>(a);                                                      \
+    }
+#define TMAC_ANYG_KERNELS(M, MODE, LPR) \
+    TMAC_ANYG_KERNEL(M, MODE, LPR, 1)   \
+    TMAC_ANYG_KERNEL(M, MODE, LPR, 2)   \
+    TMAC_ANYG_KERNEL(M, MODE, LPR, 4)   \
+    TMAC_ANYG_KERNEL(M, MODE, LPR, 8)
+#define TMAC_ANYG_MODE(M, MODE)                                                                        \
+    TMAC_ANYG_KERNELS(M, MODE, 4)                                                                      \
+    TMAC_ANYG_KERNELS(M, MODE, 8)                                                                      \
+    TMAC_ANYG_KERNELS(M, MODE, 16)                                                                     \
+    TMAC_ANYG_KERNELS(M, MODE, 32)                                                                     \
+    extern "C" __global__ __launch_bounds__(kAnyMaxDim) void tmac_##M##_any_combine(DecodeArgs a) {    \
+        any_combine_body<MODE>(a);                                                                     \
+    }
+TMAC_ANYG_MODE(decode_u, kUniform)
+TMAC_ANYG_MODE(decode_r, kRagged)
+TMAC_ANYG_MODE(layer, kLayer)
 #endif
 
 #if TMAC_IN_PART(0)

@@ -124,6 +124,8 @@ struct tmac_context {
     std::map<std::pair<int, int>, hipFunction_t> prefill_combine;  // merge of its key runs
     std::map<int, hipFunction_t> prefill_pack[2][4];          // prefill tile packing: [paged][cache type], by KV
     hipFunction_t any[3] = {};  // any-shape decode kernel by mode (shapes with no compiled kernel)
+    hipFunction_t any_group[3][4][4] = {};  // the same with GQA sharing: by mode, lanes per row 4 << i, heads 1 << j
+    hipFunction_t any_combine[3] = {};
     hipFunction_t k_rope = nullptr, k_copy = nullptr, k_pos = nullptr, k_qkv = nullptr, k_cvt16 = nullptr,
                   k_kq = nullptr, k_cvt_q8 = nullptr;
     float* ws = nullptr;
@@ -244,6 +246,7 @@ hipError_t aux_copy(tmac_context* ctx, void* dst, const void* src, size_t bytes,
 struct Kernels {
     hipFunction_t group = nullptr, head = nullptr, combine = nullptr;
     hipFunction_t hv = nullptr;      // short-context split-V head kernel (fp32 caches, not paged)
+    int any_mode = 0;
     hipFunction_t any = nullptr;     // any-shape kernel: a shape with no compiled kernel (fp32, not paged)
     int hv_split = 1;
     hipFunction_t group4 = nullptr;  // 4-wave group kernel when the size is chosen per call (fp32 caches)
@@ -271,6 +274,7 @@ int check_shape(tmac_context* ctx, int n_head, int n_kv_head, int head_dim, Kern
             if (k) {
                 *k = Kernels{};
                 k->any = ctx->any[mode];
+                k->any_mode = mode;
             }
             return TMAC_OK;
         }
@@ -524,6 +528,47 @@ int launch(tmac_context* ctx, hipFunction_t f, unsigned gx, unsigned gy, unsigne
 
 const float kQScale = (float)(1.4426950408889634 / 8.0);  // log2(e) / sqrt(64)
 
+// Any-shape decode.  head_dim a multiple of 4: the group kernel, whose 16-byte
+// loads need it; otherwise (head_dim 4 n + 2) the row kernel, one workgroup per
+// (query head, sequence).  A workgroup serves up to 8 query heads of a kv head;
+// the rows are split until the workgroups reach kAnyTargetPerCu per CU, into
+// runs of at least kAnyMinRows rows, and batches that still leave half of the
+// CUs idle serve fewer heads per workgroup (each then reads the rows through
+// L2).  Without room for the splits' partials the rows stay whole.
+constexpr int kAnyTargetPerCu = 2, kAnyMinRows = 128;
+int run_decode_any(tmac_context* ctx, hipStream_t stream, const Kernels& k, DecodeArgs& a, int n_seq, int grid_rows,
+                   int n_kv_head) {
+    a.n_kv_head = n_kv_head;
+    a.ws = nullptr;
+    a.split_len = grid_rows;
+    a.n_splits = 1;
+    const int group = a.n_head / n_kv_head;
+    int gt = 0;  // heads per workgroup: 1 << gt
+    while (gt < 3 && (1 << gt) < group) gt++;
+    auto tiles = [&] { return (group + (1 << gt) - 1) >> gt; };
+    if (a.head_dim % 4 != 0 || (int64_t)n_kv_head * group > 65535)
+        return launch(ctx, k.any, (unsigned)a.n_head, (unsigned)n_seq, tmac::kAnyWavesHost * 64, stream, &a);
+    const int64_t units = (int64_t)n_seq * n_kv_head * tiles();
+    int64_t want = std::min<int64_t>((kAnyTargetPerCu * (int64_t)ctx->n_cu + units - 1) / units,
+                                     std::min(grid_rows / kAnyMinRows, kMaxSplits));
+    if (want > 1) {
+        const int64_t len = (((int64_t)grid_rows + want - 1) / want + 31) / 32 * 32;
+        const int n_splits = (int)((grid_rows + len - 1) / len);
+        const size_t floats = (size_t)n_seq * n_splits * a.n_head * (a.head_dim + 2);
+        if (n_splits > 1 && ensure_workspace(ctx, stream, floats) == TMAC_OK) {
+            a.split_len = (int)len;
+            a.n_splits = n_splits;
+            a.ws = workspace(ctx);
+        }
+    }
+    while (gt > 0 && (int64_t)n_seq * n_kv_head * tiles() * a.n_splits * 2 <= ctx->n_cu) gt--;
+    const int n4 = a.head_dim / 4, li = n4 <= 8 ? 0 : n4 <= 16 ? 1 : n4 <= 32 ? 2 : 3;  // 4 << li lanes of 8 dims
+    int rc = launch(ctx, ctx->any_group[k.any_mode][li][gt], (unsigned)a.n_splits, (unsigned)(n_kv_head * tiles()),
+                    tmac::any_group_waves(1 << gt) * 64, stream, &a, (unsigned)n_seq);
+    if (rc || a.n_splits == 1) return rc;
+    return launch(ctx, ctx->any_combine[k.any_mode], (unsigned)a.n_head, (unsigned)n_seq, kAnyMaxDim, stream, &a);
+}
+
 // Common launch of a decode-family kernel, plus the split merge when the
 // rows are spread over more than one workgroup per sequence.
 int run_decode(tmac_context* ctx, hipStream_t stream, const Kernels& k, DecodeArgs& a, int n_seq,
@@ -533,13 +578,7 @@ int run_decode(tmac_context* ctx, hipStream_t stream, const Kernels& k, DecodeAr
     a.blocked = (int)ctx->opt_blocked;
     a.err = ctx->err;
     if (n_seq > 65535) return fail(ctx, TMAC_ERR_INVALID_ARG, "n_seq exceeds 65535");
-    if (k.any) {  // one workgroup per (query head, sequence), no split
-        a.split_len = grid_rows;
-        a.n_splits = 1;
-        a.ws = nullptr;
-        a.n_kv_head = n_kv_head;
-        return launch(ctx, k.any, (unsigned)a.n_head, (unsigned)n_seq, tmac::kAnyWavesHost * 64, stream, &a);
-    }
+    if (k.any) return run_decode_any(ctx, stream, k, a, n_seq, grid_rows, n_kv_head);
     const bool unit_grid = a.lengths || a.positions;  // ragged and paged modes
     if (k.head && use_head_kernel(ctx, n_seq, a.n_head, grid_rows)) {
         a.split_len = grid_rows;
@@ -862,9 +901,19 @@ int tmac_init(tmac_context** out, int device) {
     }
     {
         const char* any_name[3] = {"tmac_decode_u_any", "tmac_decode_r_any", "tmac_layer_any"};
-        for (int m = 0; m < 3; m++)
+        for (int m = 0; m < 3; m++) {
+            char name[64];
             if ((e = get_function(ctx, &ctx->any[m], any_name[m])) != hipSuccess)
                 return bail(hip_fail(ctx, e, any_name[m]));
+            for (int i = 0; i < 16; i++) {
+                std::snprintf(name, sizeof(name), "%s_l%d_g%d", any_name[m], 4 << (i / 4), 1 << (i % 4));
+                if ((e = get_function(ctx, &ctx->any_group[m][i / 4][i % 4], name)) != hipSuccess)
+                    return bail(hip_fail(ctx, e, name));
+            }
+            std::snprintf(name, sizeof(name), "%s_combine", any_name[m]);
+            if ((e = get_function(ctx, &ctx->any_combine[m], name)) != hipSuccess)
+                return bail(hip_fail(ctx, e, name));
+        }
     }
     if ((e = get_function(ctx, &ctx->k_rope, "tmac_rope")) != hipSuccess ||
         (e = get_function(ctx, &ctx->k_copy, "tmac_copy")) != hipSuccess ||
