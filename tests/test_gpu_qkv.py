@@ -248,3 +248,35 @@ def test_kquant_matmul_and_residual_match_oracle(ctx, qtype):
     assert ctx.matmul(qtype, rows, 896, dw, dx, dy, check=False) == tmac_attn.TMAC_ERR_INVALID_ARG
     for d in (dw, dx, dy, dh):
         d.free()
+
+
+@pytest.mark.parametrize("qtype", [oracle.Q5_0, oracle.Q8_0, oracle.Q4_K, oracle.Q6_K])
+@pytest.mark.parametrize("rows,cols", [(16387, 256), (16384, 2304), (130, 4864), (3, 8192)])
+def test_gemv_rows_and_rounds(ctx, qtype, rows, cols):
+    """Rows past the several-rows-per-wave line (256 CUs x 64; a last wave with 3 rows) and inputs
+    of several load rounds with remainders, weights at an odd multiple of 2 bytes, y = W x and
+    y += W x against the oracle on sampled rows (all rows written)."""
+    rng = np.random.default_rng(rows + cols)
+    raw = rng.integers(0, 256, (rows * (cols // (256 if qtype >= tmac_attn.TMAC_Q4_K else 32)),
+                                oracle.BLOCK_BYTES[qtype]), dtype=np.uint8)
+    sc = {oracle.Q5_0: 2e-3, oracle.Q8_0: 3e-4, oracle.Q4_K: 4e-5, oracle.Q6_K: 1e-5}[qtype]
+    for at in ([208] if qtype == oracle.Q6_K else [0, 2] if qtype == oracle.Q4_K else [0]):  # fp16 scales
+        raw[:, at:at + 2] = rng.uniform(0.5 * sc, sc, (raw.shape[0], 1)).astype(np.float16).view(np.uint8)
+    w = raw.reshape(-1)
+    x = rng.standard_normal(cols).astype(np.float32)
+    shifted = np.concatenate([np.zeros(2, np.uint8), w])
+    dw, dx, dy = ctx.upload(shifted), ctx.upload(x), ctx.empty(rows)
+    dy.fill_bytes(0xFF)
+    ctx.matmul(qtype, rows, cols, dw.ptr + 2, dx, dy)
+    got = dy.numpy()
+    assert np.all(np.isfinite(got))
+    pick = np.unique(np.concatenate([np.arange(min(rows, 9)), np.arange(max(rows - 9, 0), rows),
+                                     rng.integers(0, rows, 40)]))
+    row_bytes = w.size // rows
+    sub = np.ascontiguousarray(w.reshape(rows, row_bytes)[pick]).reshape(-1)
+    ref = oracle.matmul_q(qtype, sub, x, pick.size, cols)
+    assert_close(got[pick], ref, f"gemv type {qtype} {rows}x{cols}")
+    ctx.matmul(qtype, rows, cols, dw.ptr + 2, dx, dy, accumulate=True)
+    np.testing.assert_array_equal(dy.numpy(), got + got)
+    for d in (dw, dx, dy):
+        d.free()

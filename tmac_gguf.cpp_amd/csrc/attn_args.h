@@ -169,7 +169,8 @@ struct QkvArgs {
     int cols;
     int v_is_q8;
 };
-constexpr int kQkvWaves = 4;         // output rows per workgroup (one wave each)
+constexpr int kQkvWaves = 4;         // waves per workgroup, one output row each (large matrices: kGemvRows each)
+constexpr int kGemvRows = 4;
 
 // y = W x (+ bias) for K-quant weights: rows of cols / 256 super-blocks, Q4_K
 // (type 12, 144 bytes) or Q6_K (type 14, 210 bytes).  bias may equal y (the

@@ -1752,6 +1752,10 @@ template <bool V>
 struct BoolTag {
     static constexpr bool value = V;
 };
+template <int V>
+struct IntTag {
+    static constexpr int value = V;
+};
 constexpr int kAnyDpl = kAnyMaxDim / 32;  // dims per lane at most
 
 __device__ __forceinline__ float half_sum(float x) {  // sum over the 32 lanes of a half wave
@@ -3756,7 +3760,108 @@ TMAC_MDECODE_KERNELS(8, 1)
 // is one fused multiply-add per element, then a wave reduction, so it differs
 // from the reference's sequential sum only by rounding (wave_sum).
 
+// Weight bytes start at even offsets only; the loads are as wide as the fields
+// (16, 8 and 4 bytes at 2-byte alignment, which the memory pipeline takes), not
+// one per 16-bit word: the output head (151936 x 896, Q8_0) spent 60 us on 9
+// word loads and 4 loads of x per lane and row, 2.4 TB/s; 42 us now.
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
+typedef unsigned u32_a2 __attribute__((aligned(2)));
 __device__ __forceinline__ unsigned ld16(const uint8_t* p) { return *reinterpret_cast<const uint16_t*>(p); }
+__device__ __forceinline__ unsigned ld32(const uint8_t* p) { return *reinterpret_cast<const u32_a2*>(p); }
+
+// Half h of a block of 32 weights as loaded, and its 16 products with x added
+// to acc in the fixed order above.
+template <bool Q8>
+struct HalfBlock;
+template <>
+struct HalfBlock<true> {
+    static constexpr int kBytes = 34;
+    unsigned d;
+    u32x4 q;
+    __device__ void load(const uint8_t* blk, int h) {
+        d = ld16(blk);
+        q = *reinterpret_cast<const u32x4_a2*>(blk + 2 + 16 * h);
+    }
+    __device__ void dot(const float (&x)[16], int, float& acc) const {
+        const float df = half_bits_to_float(d);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc = __builtin_fmaf((float)(int8_t)(q[i / 4] >> (8 * (i % 4))) * df, x[i], acc);
+    }
+};
+template <>
+struct HalfBlock<false> {
+    static constexpr int kBytes = 22;
+    unsigned d, qh;
+    u32x2 q;
+    __device__ void load(const uint8_t* blk, int h) {
+        d = ld16(blk);
+        qh = ld32(blk + 2);
+        q = *reinterpret_cast<const u32x2_a2*>(blk + 6 + 8 * h);
+    }
+    __device__ void dot(const float (&x)[16], int h, float& acc) const {
+        const float df = half_bits_to_float(d);
+        const unsigned hb = qh >> (8 * h);  // bit i: element 8 h + i, bit 16 + i: element 16 + 8 h + i
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const unsigned byte = (q[i / 4] >> (8 * (i % 4))) & 0xFF;
+            const int qlo = (int)((byte & 0xF) | (((hb >> i) & 1) << 4)) - 16;
+            const int qhi = (int)((byte >> 4) | (((hb >> (i + 16)) & 1) << 4)) - 16;
+            acc = __builtin_fmaf(df * (float)qlo, x[i], acc);
+            acc = __builtin_fmaf(df * (float)qhi, x[8 + i], acc);
+        }
+    }
+};
+// The 16 inputs of half h of a block at xb: Q8_0 elements 16 h + i; Q5_0
+// elements 8 h + i, then 16 + 8 h + i.
+template <bool Q8>
+__device__ __forceinline__ void half_inputs(float (&x)[16], const float* __restrict__ xb, int h) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int at = Q8 ? 16 * h + 4 * i : (i < 2 ? 8 * h + 4 * i : 8 + 8 * h + 4 * i);
+        const float4 v = *reinterpret_cast<const float4*>(xb + at);
+        x[4 * i] = v.x; x[4 * i + 1] = v.y; x[4 * i + 2] = v.z; x[4 * i + 3] = v.w;
+    }
+}
+
+// Dot products of RW rows (the first at wrow, `stride` bytes apart; row j read
+// from row min(j, n_rows - 1)) with x, this lane's part.  The inputs are loaded
+// once for the RW rows, and the loads of kBlockRound rounds of 64 half blocks
+// are in flight together.
+template <bool Q8, int RW>
+__device__ __forceinline__ void block_rows(float (&acc)[RW], const uint8_t* __restrict__ wrow, size_t stride, int n_rows,
+                                           const float* __restrict__ x, int nb, int lane) {
+    constexpr int kBlockRound = RW == 1 ? 4 : 1;
+    const uint8_t* w[RW];
+#pragma unroll
+    for (int j = 0; j < RW; ++j) {
+        acc[j] = 0.f;
+        w[j] = wrow + (size_t)min(j, n_rows - 1) * stride;
+    }
+    const int n = 2 * nb;
+    int u = lane;
+    for (; u - lane + 64 * kBlockRound <= n && kBlockRound > 1; u += 64 * kBlockRound) {  // (wave-uniform)
+        HalfBlock<Q8> hb[kBlockRound];
+        float xv[kBlockRound][16];
+#pragma unroll
+        for (int k = 0; k < kBlockRound; ++k) {
+            const int uk = u + 64 * k;
+            hb[k].load(w[0] + (size_t)(uk >> 1) * HalfBlock<Q8>::kBytes, uk & 1);
+            half_inputs<Q8>(xv[k], x + 32 * (uk >> 1), uk & 1);
+        }
+#pragma unroll
+        for (int k = 0; k < kBlockRound; ++k) hb[k].dot(xv[k], lane & 1, acc[0]);
+    }
+    for (; u < n; u += 64) {
+        HalfBlock<Q8> hb[RW];
+        float xv[16];
+#pragma unroll
+        for (int j = 0; j < RW; ++j) hb[j].load(w[j] + (size_t)(u >> 1) * HalfBlock<Q8>::kBytes, u & 1);
+        half_inputs<Q8>(xv, x + 32 * (u >> 1), u & 1);
+#pragma unroll
+        for (int j = 0; j < RW; ++j) hb[j].dot(xv, u & 1, acc[j]);
+    }
+}
 
 extern "C" __global__ __launch_bounds__(kQkvWaves * 64) void tmac_qkv(QkvArgs a) {
     const int lane = threadIdx.x & 63;
@@ -3772,58 +3877,37 @@ extern "C" __global__ __launch_bounds__(kQkvWaves * 64) void tmac_qkv(QkvArgs a)
             if (r >= a.rows[2]) return;
         }
     }
-    const bool q8 = seg == 2 && a.v_is_q8;
     const int nb = a.cols >> 5;
-    const int bytes = q8 ? 34 : 22;
-    const uint8_t* wrow = a.w[seg] + (size_t)r * nb * bytes;
-    float acc = 0.f;
-    for (int u = lane; u < 2 * nb; u += 64) {
-        const int b = u >> 1, h = u & 1;
-        const uint8_t* blk = wrow + (size_t)b * bytes;
-        const float d = half_bits_to_float(ld16(blk));
-        const float* xb = a.x + 32 * b;
-        if (q8) {
-            const float4 x0 = *reinterpret_cast<const float4*>(xb + 16 * h);
-            const float4 x1 = *reinterpret_cast<const float4*>(xb + 16 * h + 4);
-            const float4 x2 = *reinterpret_cast<const float4*>(xb + 16 * h + 8);
-            const float4 x3 = *reinterpret_cast<const float4*>(xb + 16 * h + 12);
-            const float xv[16] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w,
-                                  x2.x, x2.y, x2.z, x2.w, x3.x, x3.y, x3.z, x3.w};
+    const float* bias = a.bias[seg];
+    const float bv = bias ? bias[r] : 0.f;
+    float acc[1];
+    if (seg == 2 && a.v_is_q8)
+        block_rows<true, 1>(acc, a.w[seg] + (size_t)r * nb * 34, 0, 1, a.x, nb, lane);
+    else
+        block_rows<false, 1>(acc, a.w[seg] + (size_t)r * nb * 22, 0, 1, a.x, nb, lane);
+    acc[0] = wave_sum(acc[0]);
+    if (lane == 0) a.y[seg][r] = bias ? acc[0] + bv : acc[0];
+}
+
+// One large matrix (the third segment): kGemvRows rows per wave, so that the
+// inputs are loaded once for them and 4 KB of weights are in flight per wave.
+template <bool Q8>
+__device__ __forceinline__ void gemv_rows_body(const QkvArgs& a) {
+    const int lane = threadIdx.x & 63;
+    const int r0 = (blockIdx.x * kQkvWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * kGemvRows;
+    if (r0 >= a.rows[2]) return;
+    const int nb = a.cols >> 5, n_rows = min(kGemvRows, a.rows[2] - r0);
+    const size_t stride = (size_t)nb * HalfBlock<Q8>::kBytes;
+    float acc[kGemvRows];
+    block_rows<Q8, kGemvRows>(acc, a.w[2] + (size_t)r0 * stride, stride, n_rows, a.x, nb, lane);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const unsigned pr = ld16(blk + 2 + 16 * h + 2 * i);
-                acc = __builtin_fmaf((float)(int8_t)(pr & 0xFF) * d, xv[2 * i], acc);
-                acc = __builtin_fmaf((float)(int8_t)(pr >> 8) * d, xv[2 * i + 1], acc);
-            }
-        } else {
-            const unsigned qh = ld16(blk + 2) | (ld16(blk + 4) << 16);
-            const float4 l0 = *reinterpret_cast<const float4*>(xb + 8 * h);
-            const float4 l1 = *reinterpret_cast<const float4*>(xb + 8 * h + 4);
-            const float4 h0 = *reinterpret_cast<const float4*>(xb + 16 + 8 * h);
-            const float4 h1 = *reinterpret_cast<const float4*>(xb + 16 + 8 * h + 4);
-            const float xl[8] = {l0.x, l0.y, l0.z, l0.w, l1.x, l1.y, l1.z, l1.w};
-            const float xh[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const unsigned pr = ld16(blk + 6 + 8 * h + 2 * i);
-#pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    const int j = 8 * h + 2 * i + t;  // element j and j + 16
-                    const unsigned byte = (pr >> (8 * t)) & 0xFF;
-                    const int qlo = (int)((byte & 0xF) | (((qh >> j) & 1) << 4)) - 16;
-                    const int qhi = (int)((byte >> 4) | (((qh >> (j + 16)) & 1) << 4)) - 16;
-                    acc = __builtin_fmaf(d * (float)qlo, xl[2 * i + t], acc);
-                    acc = __builtin_fmaf(d * (float)qhi, xh[2 * i + t], acc);
-                }
-            }
-        }
-    }
-    acc = wave_sum(acc);
-    if (lane == 0) {
-        const float* bias = a.bias[seg];
-        a.y[seg][r] = bias ? acc + bias[r] : acc;
+    for (int j = 0; j < kGemvRows; ++j) {
+        const float v = wave_sum(acc[j]);
+        if (lane == 0 && j < n_rows) a.y[2][r0 + j] = a.bias[2] ? v + a.bias[2][r0 + j] : v;
     }
 }
+extern "C" __global__ __launch_bounds__(kQkvWaves * 64) void tmac_gemv_rows_q8_0(QkvArgs a) { gemv_rows_body<true>(a); }
+extern "C" __global__ __launch_bounds__(kQkvWaves * 64) void tmac_gemv_rows_q5_0(QkvArgs a) { gemv_rows_body<false>(a); }
 
 // RoPE in place, one lane per (head, pair): tmac_gguf.cpp:992-1003 for one
 // tensor, i.e. what rope_op (metal_backend.hpp:381) dispatches.
@@ -3861,64 +3945,109 @@ extern "C" __global__ __launch_bounds__(256) void tmac_copy(CopyArgs a) {
 // expression (Q6_K: d * scale * q, exact; Q4_K: d * sc * q - dmin * m, exact
 // products and one rounding); the row sum is one FMA per element and a wave
 // reduction.
-extern "C" __global__ __launch_bounds__(kQkvWaves * 64) void tmac_matmul_kq(KqArgs a) {
+// This lane's 4 weights of a super-block as loaded, and dequantised.
+template <bool Q6>
+struct KBlock;
+template <>
+struct KBlock<true> {
+    static constexpr int kBytes = 210;
+    unsigned d, ql, qh, sc;
+    __device__ void load(const uint8_t* blk, int lane) {
+        const int half = lane >> 5, sub = (lane >> 3) & 3, l0 = 4 * (lane & 7);
+        d = ld16(blk + 208);
+        sc = blk[192 + half * 8 + (l0 >> 4) + 2 * sub];
+        ql = ld32(blk + half * 64 + l0 + ((sub & 1) ? 32 : 0));
+        qh = ld32(blk + 128 + half * 32 + l0);
+    }
+    __device__ void weights(float (&w)[4], int lane) const {
+        const int sub = (lane >> 3) & 3;
+        const float dsc = half_bits_to_float(d) * (float)(int8_t)sc;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const unsigned lb = (ql >> (8 * i)) & 0xFF;
+            const unsigned lo = sub < 2 ? (lb & 0xF) : (lb >> 4);
+            const unsigned hi = ((qh >> (8 * i)) >> (2 * sub)) & 0x3;
+            w[i] = dsc * (float)((int)((hi << 4) | lo) - 32);
+        }
+    }
+};
+template <>
+struct KBlock<false> {
+    static constexpr int kBytes = 144;
+    unsigned dd, s0, s1, s2, q;  // d | dmin << 16, the 12 bytes of 6-bit scales and mins, 4 bytes of nibbles
+    __device__ void load(const uint8_t* blk, int lane) {
+        const int sbk = lane >> 3;
+        const u32x4 hd = *reinterpret_cast<const u32x4_a2*>(blk);
+        dd = hd[0];
+        s0 = hd[1];
+        s1 = hd[2];
+        s2 = hd[3];
+        q = ld32(blk + 16 + (sbk >> 1) * 32 + 4 * (lane & 7));
+    }
+    __device__ void weights(float (&w)[4], int lane) const {
+        const int sbk = lane >> 3, sh = 8 * (sbk & 3);
+        const unsigned b0 = (s0 >> sh) & 0xFF, b1 = (s1 >> sh) & 0xFF, b2 = (s2 >> sh) & 0xFF;
+        const unsigned sc = sbk < 4 ? b0 & 63 : (b2 & 0xF) | ((b0 >> 6) << 4);
+        const unsigned m = sbk < 4 ? b1 & 63 : (b2 >> 4) | ((b1 >> 6) << 4);
+        const float dsc = half_bits_to_float(dd & 0xFFFF) * (float)sc, dm = half_bits_to_float(dd >> 16) * (float)m;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const unsigned byte = (q >> (8 * i)) & 0xFF;
+            const unsigned q4 = (sbk & 1) ? (byte >> 4) : (byte & 0xF);
+            w[i] = dsc * (float)q4 - dm;
+        }
+    }
+};
+
+// RW rows per wave; the loads of kSbRound super-blocks are in flight together.
+template <bool Q6, int RW>
+__device__ __forceinline__ void kq_body(const KqArgs& a) {
+    constexpr int kSbRound = RW == 1 ? 8 : 2;
     const int lane = threadIdx.x & 63;
-    const int r = blockIdx.x * kQkvWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (r >= a.rows) return;
-    const int nsb = a.cols >> 8;
-    const bool q6 = a.type == 14;
-    const int bytes = q6 ? 210 : 144;
-    const uint8_t* wrow = a.w + (size_t)r * nsb * bytes;
-    float acc = 0.f;
-    for (int sb = 0; sb < nsb; ++sb) {
-        const uint8_t* blk = wrow + (size_t)sb * bytes;
-        const float4 xv = *reinterpret_cast<const float4*>(a.x + 256 * sb + 4 * lane);
-        const float xs[4] = {xv.x, xv.y, xv.z, xv.w};
-        float w[4];
-        if (q6) {
-            const int half = lane >> 5, sub = (lane >> 3) & 3, l0 = 4 * (lane & 7);
-            const float d = half_bits_to_float(ld16(blk + 208));
-            const float dsc = d * (float)(int8_t)blk[192 + half * 8 + (l0 >> 4) + 2 * sub];
-            const uint8_t* ql = blk + half * 64 + l0 + ((sub & 1) ? 32 : 0);
-            const uint8_t* qh = blk + 128 + half * 32 + l0;
-            const unsigned qlw = ld16(ql) | (ld16(ql + 2) << 16);
-            const unsigned qhw = ld16(qh) | (ld16(qh + 2) << 16);
+    const int r0 = (blockIdx.x * kQkvWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * RW;
+    if (r0 >= a.rows) return;
+    const int nsb = a.cols >> 8, n_rows = min(RW, a.rows - r0);
+    const uint8_t* w[RW];
+    float acc[RW];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const unsigned lb = (qlw >> (8 * i)) & 0xFF;
-                const unsigned lo = sub < 2 ? (lb & 0xF) : (lb >> 4);
-                const unsigned hi = ((qhw >> (8 * i)) >> (2 * sub)) & 0x3;
-                w[i] = dsc * (float)((int)((hi << 4) | lo) - 32);
-            }
-        } else {
-            const int sbk = lane >> 3, q_pos = 4 * (lane & 7);
-            const float d = half_bits_to_float(ld16(blk));
-            const float dmin = half_bits_to_float(ld16(blk + 2));
-            const uint8_t* sc6 = blk + 4;
-            unsigned sc, m;
-            if (sbk < 4) {
-                sc = sc6[sbk] & 63;
-                m = sc6[sbk + 4] & 63;
-            } else {
-                sc = (sc6[sbk + 4] & 0xF) | ((sc6[sbk - 4] >> 6) << 4);
-                m = (sc6[sbk + 4] >> 4) | ((sc6[sbk] >> 6) << 4);
-            }
-            const uint8_t* qs = blk + 16 + (sbk >> 1) * 32 + q_pos;
-            const unsigned qw = ld16(qs) | (ld16(qs + 2) << 16);
-            const float dsc = d * (float)sc, dm = dmin * (float)m;
+    for (int j = 0; j < RW; ++j) {
+        acc[j] = 0.f;
+        w[j] = a.w + (size_t)(r0 + min(j, n_rows - 1)) * nsb * KBlock<Q6>::kBytes;
+    }
+    auto round = [&](int sb, auto count) {
+        constexpr int N = decltype(count)::value;
+        KBlock<Q6> kb[N][RW];
+        float4 xv[N];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const unsigned b = (qw >> (8 * i)) & 0xFF;
-                const unsigned q4 = (sbk & 1) ? (b >> 4) : (b & 0xF);
-                w[i] = dsc * (float)q4 - dm;
-            }
+        for (int k = 0; k < N; ++k) {
+            xv[k] = *reinterpret_cast<const float4*>(a.x + 256 * (sb + k) + 4 * lane);
+#pragma unroll
+            for (int j = 0; j < RW; ++j) kb[k][j].load(w[j] + (size_t)(sb + k) * KBlock<Q6>::kBytes, lane);
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc = __builtin_fmaf(w[i], xs[i], acc);
+        for (int k = 0; k < N; ++k)
+#pragma unroll
+            for (int j = 0; j < RW; ++j) {
+                float wt[4];
+                kb[k][j].weights(wt, lane);
+                acc[j] = __builtin_fmaf(wt[0], xv[k].x, acc[j]);
+                acc[j] = __builtin_fmaf(wt[1], xv[k].y, acc[j]);
+                acc[j] = __builtin_fmaf(wt[2], xv[k].z, acc[j]);
+                acc[j] = __builtin_fmaf(wt[3], xv[k].w, acc[j]);
+            }
+    };
+    int sb = 0;
+    for (; sb + kSbRound <= nsb; sb += kSbRound) round(sb, IntTag<kSbRound>{});
+    for (; sb < nsb; ++sb) round(sb, IntTag<1>{});
+#pragma unroll
+    for (int j = 0; j < RW; ++j) {
+        const float v = wave_sum(acc[j]);
+        if (lane == 0 && j < n_rows) a.y[r0 + j] = a.bias ? v + a.bias[r0 + j] : v;
     }
-    acc = wave_sum(acc);
-    if (lane == 0) a.y[r] = a.bias ? acc + a.bias[r] : acc;
 }
+extern "C" __global__ __launch_bounds__(kQkvWaves * 64) void tmac_matmul_q6_k(KqArgs a) { kq_body<true, 1>(a); }
+extern "C" __global__ __launch_bounds__(kQkvWaves * 64) void tmac_matmul_q4_k(KqArgs a) { kq_body<false, 1>(a); }
+extern "C" __global__ __launch_bounds__(kQkvWaves * 64) void tmac_gemv_rows_q4_k(KqArgs a) { kq_body<false, kGemvRows>(a); }
 
 // Fills a 16-bit cache from fp32 values, rounding to nearest even.
 extern "C" __global__ __launch_bounds__(256) void tmac_cvt16(CvtArgs a) {

@@ -127,7 +127,9 @@ struct tmac_context {
     hipFunction_t any_group[3][4][4] = {};  // the same with GQA sharing: by mode, lanes per row 4 << i, heads 1 << j
     hipFunction_t any_combine[3] = {};
     hipFunction_t k_rope = nullptr, k_copy = nullptr, k_pos = nullptr, k_qkv = nullptr, k_cvt16 = nullptr,
-                  k_kq = nullptr, k_cvt_q8 = nullptr;
+                  k_cvt_q8 = nullptr;
+    // quantized GEMV of a large matrix; K-quants: [Q6_K][large matrix] (Q6_K: one kernel for both)
+    hipFunction_t k_gemv_q8 = nullptr, k_gemv_q5 = nullptr, k_kq[2][2] = {};
     float* ws = nullptr;
     size_t ws_floats = 0;
     int* err = nullptr;
@@ -920,7 +922,11 @@ int tmac_init(tmac_context** out, int device) {
         (e = get_function(ctx, &ctx->k_pos, "tmac_pos_update")) != hipSuccess ||
         (e = get_function(ctx, &ctx->k_qkv, "tmac_qkv")) != hipSuccess ||
         (e = get_function(ctx, &ctx->k_cvt16, "tmac_cvt16")) != hipSuccess ||
-        (e = get_function(ctx, &ctx->k_kq, "tmac_matmul_kq")) != hipSuccess ||
+        (e = get_function(ctx, &ctx->k_gemv_q8, "tmac_gemv_rows_q8_0")) != hipSuccess ||
+        (e = get_function(ctx, &ctx->k_gemv_q5, "tmac_gemv_rows_q5_0")) != hipSuccess ||
+        (e = get_function(ctx, &ctx->k_kq[0][0], "tmac_matmul_q4_k")) != hipSuccess ||
+        (e = get_function(ctx, &ctx->k_kq[0][1], "tmac_gemv_rows_q4_k")) != hipSuccess ||
+        (e = get_function(ctx, &ctx->k_kq[1][0], "tmac_matmul_q6_k")) != hipSuccess ||
         (e = get_function(ctx, &ctx->k_cvt_q8, "tmac_cvt_q8")) != hipSuccess)
         return bail(hip_fail(ctx, e, "hipModuleGetFunction"));
     if ((e = hipStreamCreateWithFlags(&ctx->aux, hipStreamNonBlocking)) != hipSuccess)
@@ -1588,6 +1594,16 @@ int tmac_elem_op(tmac_context* ctx, tmac_stream stream, int op, float* data, con
     return launch(ctx, ctx->k_copy, (unsigned)((dim + 255) / 256), 1, 256, (hipStream_t)stream, &a);
 }
 
+// GEMV grids: one output row per wave, or kGemvRows in a large matrix, whose
+// rows still give every SIMD several waves (Q8_0, 4 rows a wave against 1, us:
+// 32000 x 1024 14.8 -> 10.0, 16000 x 1024 equal).  Q6_K stays at one row: its
+// loads are 4 bytes a lane whatever the rows (32000 x 4864 73 us, 84 with 4).
+static bool large_gemv(const tmac_context* ctx, int rows) { return rows >= 64 * ctx->n_cu; }
+static unsigned gemv_grid(int64_t rows, bool large) {
+    const int per = kQkvWaves * (large ? tmac::kGemvRows : 1);
+    return (unsigned)((rows + per - 1) / per);
+}
+
 static int qkv_common(tmac_context* ctx, hipStream_t stream, const void* w_q, const void* w_k, const void* w_v,
                       const float* x, const float* b_q, const float* b_k, const float* b_v, float* y_q,
                       float* y_k, float* y_v, int q_rows, int k_rows, int v_rows, int cols, int v_is_q8) {
@@ -1608,7 +1624,10 @@ static int qkv_common(tmac_context* ctx, hipStream_t stream, const void* w_q, co
     if ((rc = set_device(ctx))) return rc;
     QkvArgs a{{(const uint8_t*)w_q, (const uint8_t*)w_k, (const uint8_t*)w_v}, x, {b_q, b_k, b_v},
               {y_q, y_k, y_v}, {q_rows, k_rows, v_rows}, cols, v_is_q8 ? 1 : 0};
-    return launch(ctx, ctx->k_qkv, (unsigned)((total + kQkvWaves - 1) / kQkvWaves), 1, kQkvWaves * 64, stream, &a);
+    if (total == v_rows && large_gemv(ctx, v_rows))
+        return launch(ctx, v_is_q8 ? ctx->k_gemv_q8 : ctx->k_gemv_q5, gemv_grid(v_rows, true), 1, kQkvWaves * 64, stream,
+                      &a);
+    return launch(ctx, ctx->k_qkv, gemv_grid(total, false), 1, kQkvWaves * 64, stream, &a);
 }
 
 int tmac_fused_qkv_op(tmac_context* ctx, tmac_stream stream, const void* w_q, const void* w_k, const void* w_v,
@@ -1644,8 +1663,8 @@ static int matmul_common(tmac_context* ctx, hipStream_t stream, int qtype, int r
         if (rows == 0) return TMAC_OK;
         if ((rc = set_device(ctx))) return rc;
         KqArgs a{(const uint8_t*)w, x, accumulate ? y : nullptr, y, rows, cols, qtype};
-        return launch(ctx, ctx->k_kq, (unsigned)((rows + kQkvWaves - 1) / kQkvWaves), 1, kQkvWaves * 64, stream,
-                      &a);
+        const bool large = qtype == TMAC_Q4_K && large_gemv(ctx, rows);
+        return launch(ctx, ctx->k_kq[qtype == TMAC_Q6_K][large], gemv_grid(rows, large), 1, kQkvWaves * 64, stream, &a);
     }
     return qkv_common(ctx, stream, nullptr, nullptr, w, x, nullptr, nullptr, accumulate ? y : nullptr, nullptr,
                       nullptr, y, 0, 0, rows, cols, qtype == TMAC_Q8_0);
