@@ -808,3 +808,49 @@ def test_decode_q8_mfma_shapes(ctx, g, kv):
     ref = oracle.attention_ragged(q, kw, vw, offs, lens, nh, kv, HD, n_threads=8)
     assert_close(dout.numpy(), ref, f"q8 ragged g={g} kv={kv}")
     assert ctx.check_device_error() == 0
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("n_seq,max_len", [(96, 700), (193, 1000), (300, 530), (511, 64)])
+def test_units_two_per_cu(ctx, dt, n_seq, max_len):
+    """Ragged and paged decode on 16-bit caches with the row-count hint, at sequence counts where
+    the splits aim at two workgroups per CU (96 to 511 sequences on 256 CUs): equal parts of the
+    longest sequence, lengths 0 and 1 and max_len among them, against the oracle."""
+    code = {"bf16": tmac_attn.TMAC_KV_BF16, "f16": tmac_attn.TMAC_KV_F16}[dt]
+    rng = np.random.default_rng(n_seq + max_len)
+    lens = rng.integers(0, max_len + 1, n_seq).astype(np.int32)
+    lens[:4] = [max_len, 0, 1, max_len - 1]
+    pages = (lens.astype(np.int64) + 15) // 16
+    n_pages, max_pages = int(pages.sum()) + 1, (max_len + 15) // 16
+    perm, table, at = rng.permutation(n_pages).astype(np.int32), np.zeros((n_seq, max_pages), np.int32), 0
+    for s in range(n_seq):
+        table[s, :pages[s]] = perm[at:at + pages[s]]
+        at += int(pages[s])
+    q = rng.standard_normal((n_seq, 14 * 64), dtype=np.float32)
+    pool = [rng.standard_normal((n_pages * 16, 128), dtype=np.float32).astype(np.float16) for _ in range(2)]
+    if dt == "bf16":  # fp16 values cut to bf16's 8 bits: exact in both types
+        bits = [(x.astype(np.float32).view(np.uint32) >> 16).astype(np.uint16) for x in pool]
+        wide = [(b.astype(np.uint32) << 16).view(np.float32) for b in bits]
+    else:
+        bits, wide = [x.view(np.uint16) for x in pool], [x.astype(np.float32) for x in pool]
+    rows = np.concatenate([np.arange(0)] + [table[s, np.arange(lens[s]) // 16].astype(np.int64) * 16 + np.arange(lens[s]) % 16
+                                            for s in range(n_seq)]).astype(np.int64)
+    offs = np.concatenate([[0], np.cumsum(lens[:-1], dtype=np.int64)]).astype(np.int64)
+    kr, vr = (np.ascontiguousarray(x[rows]) for x in wide)
+    nz = lens > 0
+    ref = np.zeros((n_seq, 14 * 64), np.float32)
+    ref[nz] = oracle.attention_ragged(q[nz], kr, vr, offs[nz], lens[nz], 14, 2, 64, n_threads=8)
+    d = [ctx.upload(x) for x in (q, *bits, table, lens, *(np.ascontiguousarray(b[rows]) for b in bits), offs)]
+    dq, dk, dv, dtab, dlen, dkr, dvr, doff = d
+    dout = ctx.empty((n_seq, 14 * 64))
+    total = int(lens.sum())
+    dout.fill_bytes(0xFF)
+    ctx.decode_paged(dq, dk, dv, n_pages, dtab, max_pages, dlen, dout, n_seq, 14, 2, 64, max_len, total_rows=total,
+                     kv_dtype=code)
+    assert_close(dout.numpy(), ref, f"paged {dt} {n_seq}x{max_len}")
+    dout.fill_bytes(0xFF)
+    ctx.decode_ragged(dq, dkr, dvr, doff, dlen, dout, n_seq, 14, 2, 64, max_len, total_rows=total, kv_dtype=code)
+    assert_close(dout.numpy(), ref, f"ragged {dt} {n_seq}x{max_len}")
+    for x in d + [dout]:
+        x.free()
+    assert ctx.check_device_error() == 0

@@ -254,6 +254,7 @@ struct Kernels {
     hipFunction_t group4 = nullptr;  // 4-wave group kernel when the size is chosen per call (fp32 caches)
     int head_waves = 16;
     int group_waves = 8;
+    bool two_per_cu = false;         // two workgroups of the group kernel fit a CU
 };
 
 // Validates the attention shape shared by every decode entry point and picks
@@ -322,6 +323,7 @@ int check_shape(tmac_context* ctx, int n_head, int n_kv_head, int head_dim, Kern
             if (f != tab.end()) {
                 k->group = f->second;
                 k->group_waves = dt == TMAC_KV_Q8_0 ? tmac::kMWavesQ8Host : tmac::kMWaves16Host;
+                k->two_per_cu = dt != TMAC_KV_Q8_0;
             }
         }
     }
@@ -337,7 +339,7 @@ int check_shape(tmac_context* ctx, int n_head, int n_kv_head, int head_dim, Kern
 // knows it) the split length is total/target instead, so the workgroups that
 // actually have rows come close to one per CU whatever the length mix.
 void choose_split(const tmac_context* ctx, int waves, int n_seq, int n_pos, int n_kv_head, int* split_len,
-                  int* n_splits, int64_t total_rows = 0, int align = 1) {
+                  int* n_splits, int64_t total_rows = 0, int align = 1, bool two_per_cu = false) {
     // `align`: split lengths are also a multiple of it (paged caches: the
     // 16-row page, which the MFMA decode's tiles and the group kernel's steps
     // must not straddle).
@@ -347,6 +349,20 @@ void choose_split(const tmac_context* ctx, int waves, int n_seq, int n_pos, int 
     const int64_t target_groups = ctx->opt_target_groups > 0 ? ctx->opt_target_groups : (int64_t)ctx->n_cu;
     if (ctx->opt_split_len > 0) {
         len = (int)(((ctx->opt_split_len + round - 1) / round) * round);
+    } else if (total_rows > 0 && two_per_cu && 8 * (int64_t)n_seq >= 3 * target_groups &&
+               2 * target_groups > n_seq) {
+        // The 4-wave MFMA decode (bf16 / fp16 caches) holds two workgroups on
+        // a CU.  With a sequence for every second or third CU or more, one
+        // unit per CU leaves too few units to even out the lengths: two per
+        // CU, the longest sequence cut into equal parts.  Lengths U[1, L],
+        // bf16, us: 128 x 4096 32.1 -> 29.4, 193 x 4096 55.0 -> 44.5, 300 x
+        // 2000 45.9 -> 37.8; below that line nothing gained (64 x 16384 56.7,
+        // 59.2), and the 8-wave Q8_0 kernel, one workgroup per CU, is mixed
+        // (193 x 4096 45.9 -> 39.1, 220 x 3000 35.9 -> 37.7, 128 x 4096 31.2
+        // -> 31.9) and keeps one unit per CU.
+        const int64_t per = (total_rows + (2 * target_groups - n_seq) - 1) / (2 * target_groups - n_seq);
+        const int64_t parts = (n_pos + per - 1) / per;
+        len = (int)(((n_pos + parts - 1) / parts + round - 1) / round * round);
     } else if (total_rows > 0 && target_groups > n_seq) {
         const int64_t per = (total_rows + (target_groups - n_seq) - 1) / (target_groups - n_seq);
         len = (int)std::min<int64_t>(((per + round - 1) / round) * round, (int64_t)rounds * round);
@@ -599,7 +615,7 @@ int run_decode(tmac_context* ctx, hipStream_t stream, const Kernels& k, DecodeAr
     }
     int split_len = 0, n_splits = 0;
     choose_split(ctx, waves, n_seq, grid_rows, n_kv_head, &split_len, &n_splits, total_rows,
-                 a.block_table ? kPageRows : 1);
+                 a.block_table ? kPageRows : 1, k.two_per_cu);
     a.split_len = split_len;
     a.n_splits = n_splits;
     if (n_splits > 1) {
