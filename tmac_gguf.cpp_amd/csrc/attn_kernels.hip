@@ -2506,10 +2506,6 @@ __device__ __forceinline__ int prefill_stages(const PrefillArgs& a, int b) {
 // answer (lane l takes block l of a round of 64; blocks number a few per CU
 // where keys are split).
 __device__ __forceinline__ bool prefill_unit(const PrefillArgs& a, int rank, int& qblk, int& part, int& n_act) {
-    if (a.split == 0) {
-        qblk = a.n_qblk - 1 - rank;
-        return qblk >= 0;
-    }
     const int lane = threadIdx.x & 63;
     int base = 0;
     for (int r0 = 0; r0 < a.n_qblk; r0 += 64) {
@@ -2530,7 +2526,10 @@ __device__ __forceinline__ bool prefill_unit(const PrefillArgs& a, int rank, int
     return false;
 }
 
-template <int G, int KV>
+// RUNS: units are key runs of the blocks (a.split > 0); otherwise whole blocks,
+// in a kernel without the run code (4 x 512 queries on 1536 rows: 37.4 us with
+// it, 37.0 without).
+template <int G, int KV, bool RUNS>
 __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
     constexpr int NH = KV * G;
     constexpr int QB = kPrefillQueries, KT = kPrefillKeys, NT = kPrefillStageTiles;
@@ -2541,15 +2540,15 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
     const int pair = wave & 3, part = wave >> 2;  // head pair, half of the stage (two tiles)
 
     const int sk = blockIdx.x % a.n_sk;  // (sequence, kv head)
-    int qblk, part_idx = 0, n_act = 1;
-    if (!prefill_unit(a, blockIdx.x / a.n_sk, qblk, part_idx, n_act)) return;
+    int qblk = a.n_qblk - 1 - (int)(blockIdx.x / a.n_sk), part_idx = 0, n_act = 1;
+    if (RUNS && !prefill_unit(a, blockIdx.x / a.n_sk, qblk, part_idx, n_act)) return;
     const int seq = sk / KV, kv = sk - seq * KV;
     const int q0 = qblk * QB;
     const int q_last = min(q0 + QB, a.n_q) - 1;
     const int kmax = a.prefix_len + q_last;  // last key any query of the block attends
     const int n_tiles = kmax / KT + 1;
-    const int st_first = part_idx * a.split;
-    const int n_stages = a.split ? min(st_first + a.split, (n_tiles + NT - 1) / NT) : (n_tiles + NT - 1) / NT;
+    const int st_first = RUNS ? part_idx * a.split : 0;
+    const int n_stages = RUNS ? min(st_first + a.split, (n_tiles + NT - 1) / NT) : (n_tiles + NT - 1) / NT;
     const __bf16* slab = reinterpret_cast<const __bf16*>(a.packed) + (size_t)sk * a.n_tp * kPrefillTileElems;
 
     // Two stage buffers as separate objects, so that the compiler sees that a
@@ -2789,10 +2788,10 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
         // One unit per block: m[hh] is finite (part 0 holds tile 0, whose key 0 every query sees).  A later
         // run of keys may hold none that an early query of the block sees: weights 0, partial (-inf, 0, 0).
         const float mx = fmaxf(m[hh], m1);
-        const float a0 = (m[hh] == kNegInf) ? 0.f : fast_exp2((m[hh] - mx) * c);
+        const float a0 = (RUNS && m[hh] == kNegInf) ? 0.f : fast_exp2((m[hh] - mx) * c);
         const float a1 = (m1 == kNegInf) ? 0.f : fast_exp2((m1 - mx) * c);
         const float ls = a0 * l[hh] + a1 * l1;
-        if (n_act > 1) {  // a run's partial, in the accumulators' own layout (256-byte stores)
+        if (RUNS && n_act > 1) {  // a run's partial, in the accumulators' own layout (256-byte stores)
             float* pp = a.part + ((((size_t)sk * a.n_qblk + qblk) * a.n_parts + part_idx) * G + hl[hh]) *
                                      kPrefillPartFloats + lane;
 #pragma unroll

@@ -121,7 +121,7 @@ struct tmac_context {
     // MFMA decode (bf16, fp16, Q8_0): uniform, ragged, paged, layer, paged layer
     std::map<std::pair<int, int>, hipFunction_t> mdecode[kNarrowTypes][5];
     std::map<std::pair<int, int>, hipFunction_t> prefill;     // chunked prefill, (G, KV)
-    std::map<std::pair<int, int>, hipFunction_t> prefill_combine;  // merge of its key runs
+    std::map<std::pair<int, int>, hipFunction_t> prefill_runs, prefill_combine;  // over key runs, and their merge
     std::map<int, hipFunction_t> prefill_pack[2][4];          // prefill tile packing: [paged][cache type], by KV
     hipFunction_t any[3] = {};  // any-shape decode kernel by mode (shapes with no compiled kernel)
     hipFunction_t any_group[3][4][4] = {};  // the same with GQA sharing: by mode, lanes per row 4 << i, heads 1 << j
@@ -900,6 +900,10 @@ int tmac_init(tmac_context** out, int device) {
                 if ((e = get_function(ctx, &f, name)) != hipSuccess)
                     return bail(hip_fail(ctx, e, name));
                 ctx->prefill[{sh[0], sh[1]}] = f;
+                std::snprintf(name, sizeof(name), "tmac_prefill_runs_g%d_kv%d", sh[0], sh[1]);
+                if ((e = get_function(ctx, &f, name)) != hipSuccess)
+                    return bail(hip_fail(ctx, e, name));
+                ctx->prefill_runs[{sh[0], sh[1]}] = f;
                 std::snprintf(name, sizeof(name), "tmac_prefill_combine_g%d_kv%d", sh[0], sh[1]);
                 if ((e = get_function(ctx, &f, name)) != hipSuccess)
                     return bail(hip_fail(ctx, e, name));
@@ -1365,7 +1369,8 @@ static PrefillPlan prefill_plan(const tmac_context* ctx, int n_sk, int group, in
 static int launch_prefill(tmac_context* ctx, hipStream_t stream, int n_head, int n_kv_head, const PrefillPlan& plan,
                    PrefillArgs& a) {
     const std::pair<int, int> key{n_head / n_kv_head, n_kv_head};
-    int rc = launch(ctx, ctx->prefill.at(key), (unsigned)plan.n_blocks, 1, kPrefillWaves * 64, stream, &a);
+    int rc = launch(ctx, (plan.split ? ctx->prefill_runs : ctx->prefill).at(key), (unsigned)plan.n_blocks, 1,
+                    kPrefillWaves * 64, stream, &a);
     if (rc || !plan.split) return rc;
     return launch(ctx, ctx->prefill_combine.at(key), (unsigned)((int64_t)a.n_sk * a.n_qblk * key.first), 1, 256, stream,
                   &a);
