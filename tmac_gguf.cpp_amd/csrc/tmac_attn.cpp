@@ -347,22 +347,26 @@ void choose_split(const tmac_context* ctx, int waves, int n_seq, int n_pos, int 
     const int rounds = (n_pos + round - 1) / round;
     int len;
     const int64_t target_groups = ctx->opt_target_groups > 0 ? ctx->opt_target_groups : (int64_t)ctx->n_cu;
-    if (ctx->opt_split_len > 0) {
-        len = (int)(((ctx->opt_split_len + round - 1) / round) * round);
-    } else if (total_rows > 0 && two_per_cu && 8 * (int64_t)n_seq >= 3 * target_groups &&
-               2 * target_groups > n_seq) {
-        // The 4-wave MFMA decode (bf16 / fp16 caches) holds two workgroups on
-        // a CU.  With a sequence for every second or third CU or more, one
-        // unit per CU leaves too few units to even out the lengths: two per
-        // CU, the longest sequence cut into equal parts.  Lengths U[1, L],
-        // bf16, us: 128 x 4096 32.1 -> 29.4, 193 x 4096 55.0 -> 44.5, 300 x
-        // 2000 45.9 -> 37.8; below that line nothing gained (64 x 16384 56.7,
-        // 59.2), and the 8-wave Q8_0 kernel, one workgroup per CU, is mixed
-        // (193 x 4096 45.9 -> 39.1, 220 x 3000 35.9 -> 37.7, 128 x 4096 31.2
-        // -> 31.9) and keeps one unit per CU.
+    // The 4-wave MFMA decode (bf16 / fp16 caches) holds two workgroups on a CU.
+    // With a sequence for every second or third CU or more, one unit per CU
+    // leaves too few units to even out the lengths: two per CU, the longest
+    // sequence cut into equal parts.  Lengths U[1, L], bf16, us: 128 x 4096
+    // 32.1 -> 29.4, 193 x 4096 55.0 -> 44.5, 300 x 2000 45.9 -> 37.8; below
+    // that line nothing gained (64 x 16384 56.7, 59.2), and the 8-wave Q8_0
+    // kernel, one workgroup per CU, is mixed (193 x 4096 45.9 -> 39.1, 220 x
+    // 3000 35.9 -> 37.7, 128 x 4096 31.2 -> 31.9) and keeps one unit per CU.
+    // Lengths so unequal that this would take more than 3.5 slots per CU keep
+    // the other rules, so the partials fit the workspace a context starts with.
+    int64_t equal_parts = 0;
+    if (total_rows > 0 && two_per_cu && 8 * (int64_t)n_seq >= 3 * target_groups && 2 * target_groups > n_seq) {
         const int64_t per = (total_rows + (2 * target_groups - n_seq) - 1) / (2 * target_groups - n_seq);
         const int64_t parts = (n_pos + per - 1) / per;
-        len = (int)(((n_pos + parts - 1) / parts + round - 1) / round * round);
+        if (2 * parts * n_seq <= 7 * target_groups) equal_parts = parts;
+    }
+    if (ctx->opt_split_len > 0) {
+        len = (int)(((ctx->opt_split_len + round - 1) / round) * round);
+    } else if (equal_parts > 0) {
+        len = (int)(((n_pos + equal_parts - 1) / equal_parts + round - 1) / round * round);
     } else if (total_rows > 0 && target_groups > n_seq) {
         const int64_t per = (total_rows + (target_groups - n_seq) - 1) / (target_groups - n_seq);
         len = (int)std::min<int64_t>(((per + round - 1) / round) * round, (int64_t)rounds * round);
