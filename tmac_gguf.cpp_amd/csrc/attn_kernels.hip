@@ -2870,7 +2870,11 @@ __device__ __forceinline__ void prefill_combine_body(const PrefillArgs& a) {
 #define TMAC_PREFILL_KERNEL(G, KV)                                                                    \
     extern "C" __global__ __launch_bounds__(kPrefillWaves * 64) void tmac_prefill_g##G##_kv##KV(      \
         PrefillArgs a) {                                                                              \
-        prefill_body<G, KV>(a);                                                                       \
+        prefill_body<G, KV, false>(a);                                                                \
+    }                                                                                                 \
+    extern "C" __global__ __launch_bounds__(kPrefillWaves * 64) void tmac_prefill_runs_g##G##_kv##KV( \
+        PrefillArgs a) {                                                                              \
+        prefill_body<G, KV, true>(a);                                                                 \
     }                                                                                                 \
     extern "C" __global__ __launch_bounds__(256) void                           \
         tmac_prefill_combine_g##G##_kv##KV(PrefillArgs a) {                                           \
