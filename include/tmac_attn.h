@@ -230,7 +230,8 @@ int tmac_attention_decode_ragged(tmac_context* ctx, tmac_stream stream, const fl
  * process ends, instead of the context's growable workspace, and the call never calls hipMalloc or
  * hipFree.  A call whose schedule needs more than TMAC_SCRATCH_BYTES of partials launches nothing and
  * returns TMAC_ERR_CAPACITY (at 14 query heads: stream-K batches up to about 4,000 sequences, unit-grid
- * batches up to n_seq * splits = 4,500).  Every call on one GPU shares that GPU's array (all contexts
+ * batches up to n_seq * splits = 4,500); a shape without compiled kernels then keeps its rows
+ * unsplit instead.  Every call on one GPU shares that GPU's array (all contexts
  * and streams): calls that overlap on one GPU race.  No part of it needs to start at zero. */
 #define TMAC_SCRATCH_BYTES (16u << 20)
 int tmac_attention_decode_ragged_noalloc(tmac_context* ctx, tmac_stream stream, const float* q,
@@ -423,7 +424,7 @@ enum tmac_kernel_choice {
 };
 int tmac_set_option(tmac_context* ctx, int option, int64_t value);
 /* Rows per workgroup and splits the next decode with this shape would use
- * (*n_splits = 0 means the head kernel). */
+ * (*n_splits = 0 means the head kernel, or a shape without compiled kernels). */
 int tmac_query_split(tmac_context* ctx, int n_seq, int n_pos, int n_head, int n_kv_head, int* split_len,
                      int* n_splits);
 /* Reads and clears the device error word (bit 0: bad device-side position, bit 1: ragged or paged length

@@ -1738,8 +1738,10 @@ __device__ __forceinline__ void combine_sk_body(const DecodeArgs& a) {
 // fp32 caches): runtime n_head, n_kv_head (n_head a multiple of it) and any
 // even head_dim up to kAnyMaxDim, as the reference's kernel_attn accepts any
 // group and head_dim (kernel_attn.metal:7-60, chosen by attention_op when
-// head_dim != 64, metal_backend.hpp:416-452).  grid = (query head, sequence),
-// one split, kAnyWaves waves.  A wave step covers 2 rows: lanes 0..31 one
+// head_dim != 64, metal_backend.hpp:416-452).  Row kernel, for the head_dims
+// that are not a multiple of 4 (the others take the group kernel below, which
+// needs 16-byte loads).  grid = (query head, sequence), one split, kAnyWaves
+// waves.  A wave step covers 2 rows: lanes 0..31 one
 // row, lanes 32..63 the next; lane c of a half holds dims c, c + 32, ...
 // (4-byte loads, 128 contiguous bytes per row per load).  q.k is summed over
 // the 32 lanes of a half; the online softmax keeps one running max per wave
@@ -3758,15 +3760,16 @@ TMAC_MDECODE_KERNELS(8, 1)
 // matrices of a layer in one launch, one wave per output row.  Lane u of a row
 // takes half of block u / 2: for Q5_0 the elements 8h + i and 16 + 8h + i
 // (i < 8; byte 8h + i of qs holds both nibbles), for Q8_0 the elements 16h + i
-// (i < 16).  Every block field sits at an even offset, so the weights are read
-// as 16-bit words.  The dequantised weight d * q is exact in fp32; the row sum
+// (i < 16).  The dequantised weight d * q is exact in fp32; the row sum
 // is one fused multiply-add per element, then a wave reduction, so it differs
 // from the reference's sequential sum only by rounding (wave_sum).
 
 // Weight bytes start at even offsets only; the loads are as wide as the fields
 // (16, 8 and 4 bytes at 2-byte alignment, which the memory pipeline takes), not
 // one per 16-bit word: the output head (151936 x 896, Q8_0) spent 60 us on 9
-// word loads and 4 loads of x per lane and row, 2.4 TB/s; 42 us now.
+// word loads and 4 loads of x per lane and row, 2.4 TB/s; 40 us, 3.6 TB/s, now
+// (what is left is not the misalignment: word-aligned loads with byte shifts
+// take the same time).
 typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
 typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
 typedef unsigned u32_a2 __attribute__((aligned(2)));
@@ -3943,11 +3946,11 @@ extern "C" __global__ __launch_bounds__(256) void tmac_copy(CopyArgs a) {
 // K-quant GEMV (matmul_q4_k / matmul_q6_k, metal_backend.hpp:340-350;
 // dequantisation tmac_gguf.cpp:330-397): one wave per output row, lane l takes
 // elements 4l .. 4l+3 of each 256-weight super-block, which share one sub-block
-// scale (and, for Q4_K, one min).  Super-blocks start at even offsets, so their
-// bytes are read as 16-bit words.  Each dequantised weight is the reference's
+// scale (and, for Q4_K, one min).  Each dequantised weight is the reference's
 // expression (Q6_K: d * scale * q, exact; Q4_K: d * sc * q - dmin * m, exact
 // products and one rounding); the row sum is one FMA per element and a wave
-// reduction.
+// reduction.  Latency-bound where the rows are few: the loads of 8 super-blocks
+// are in flight together (896 x 4864: Q4_K 8.2 -> 4.1 us, Q6_K 6.1 -> 4.3).
 // This lane's 4 weights of a super-block as loaded, and dequantised.
 template <bool Q6>
 struct KBlock;
