@@ -200,3 +200,62 @@ def test_sequence_count_limit(ctx):
     d = ctx.empty(64)
     rc = ctx.decode_batched(d, d, d, d, 65536, NH, NKV, HD, 16, 16, check=False)
     assert rc == tmac_attn.TMAC_ERR_INVALID_ARG
+
+
+@pytest.mark.parametrize("entry", ["ragged", "paged", "layer_paged"])
+@pytest.mark.parametrize("dt", [tmac_attn.TMAC_KV_F32, tmac_attn.TMAC_KV_BF16, tmac_attn.TMAC_KV_Q8_0])
+def test_length_bound_is_exact(ctx, dt, entry):
+    """A sequence one row longer than max_len gives NaN and error bit 1 whatever the split length
+    (the last split of 1,000 rows ends past row 1,000 on every unit-grid kernel), as does one of
+    2^31 - 1 rows; sequences of up to max_len rows keep their results.  The rows and block-table
+    entries past max_len are allocated."""
+    max_len, n_seq, cap = 1000, 5, 1152
+    long_ = 1 << 31 if entry != "layer_paged" else max_len + 100
+    lens = np.array([max_len, max_len + 1, 40, long_ - 1, 1], np.int64).astype(np.int32)
+    row = {tmac_attn.TMAC_KV_F32: KVD * 4, tmac_attn.TMAC_KV_BF16: KVD * 2, tmac_attn.TMAC_KV_Q8_0: NKV * 68}[dt]
+    q = oracle.normal(3400, (n_seq, NH * HD))
+    dq, dout = ctx.upload(q), ctx.empty((n_seq, NH * HD))
+    pool = []
+    for i in range(2):
+        src = ctx.upload(oracle.normal(3401 + i, (n_seq * cap, KVD)))
+        if dt == tmac_attn.TMAC_KV_F32:
+            pool.append(src)
+        else:
+            pool.append(ctx.empty(n_seq * cap * row // 4))
+            ctx.kv_convert(dt, src, pool[i], n_seq * cap * KVD)
+    dk, dv = pool
+    doff, dlen = ctx.upload(np.arange(n_seq, dtype=np.int64) * cap), ctx.upload(lens)
+    dtab = ctx.upload(np.arange(n_seq * cap // PR, dtype=np.int32).reshape(n_seq, cap // PR))
+    dpos = ctx.upload(lens - 1)
+    dkn, dvn = ctx.upload(oracle.normal(3403, (n_seq, KVD))), ctx.upload(oracle.normal(3404, (n_seq, KVD)))
+
+    def call(bound):
+        dout.fill_bytes(0x3F)
+        if entry == "ragged":
+            ctx.decode_ragged(dq, dk, dv, doff, dlen, dout, n_seq, NH, NKV, HD, bound, kv_dtype=dt)
+        elif entry == "paged":
+            ctx.decode_paged(dq, dk, dv, n_seq * cap // PR, dtab, cap // PR, dlen, dout, n_seq, NH, NKV, HD, bound,
+                             kv_dtype=dt)
+        else:
+            ctx.layer_attention_paged(dq, dkn, dvn, dk, dv, n_seq * cap // PR, dtab, cap // PR, dpos, dout, n_seq, NH,
+                                      NKV, HD, bound, 1e6, kv_dtype=dt)
+        return dout.numpy()
+
+    ctx.set_option(tmac_attn.TMAC_OPT_STREAM_K, 0)
+    ctx.set_option(tmac_attn.TMAC_OPT_KERNEL, tmac_attn.TMAC_KERNEL_GROUP)
+    try:
+        for split_len in (0, 96):
+            ctx.set_option(tmac_attn.TMAC_OPT_SPLIT_LEN, split_len)
+            got = call(max_len)
+            assert ctx.check_device_error() == tmac_attn.TMAC_ERR_DEVICE_FAULT
+            assert np.all(np.isnan(got[[1, 3]])), f"split length {split_len}"
+            ref = call(max_len + 2)
+            assert ctx.check_device_error() == tmac_attn.TMAC_ERR_DEVICE_FAULT
+            assert np.all(np.isfinite(ref[1])) and np.all(np.isnan(ref[3]))
+            assert_close(got[[0, 2, 4]], ref[[0, 2, 4]], f"sequences within max_len, split length {split_len}")
+    finally:
+        ctx.set_option(tmac_attn.TMAC_OPT_SPLIT_LEN, 0)
+        ctx.set_option(tmac_attn.TMAC_OPT_KERNEL, 0)
+        ctx.set_option(tmac_attn.TMAC_OPT_STREAM_K, 1)
+    for d in (dq, dout, dk, dv, doff, dlen, dtab, dpos, dkn, dvn):
+        d.free()

@@ -231,3 +231,38 @@ def test_any_shape_splits(ctx, nh, nkv, hd, n_seq, max_len):
     for d in (dq, dk, dv, do, dl, dout, pos_dev, dkn, dvn, dkc, dvc):
         d.free()
     assert ctx.check_device_error() == 0
+
+
+@pytest.mark.parametrize("nh,nkv,hd", [(14, 2, 128), (8, 8, 80), (9, 3, 66)])
+@pytest.mark.parametrize("n_seq", [1, 6])
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_any_shape_length_bound_is_exact(ctx, nh, nkv, hd, n_seq, noalloc):
+    """A sequence one row longer than max_len gives NaN and error bit 1, whatever the number and
+    length of the splits (1,000 rows: 7 splits of 160 at 14 / 2 heads), as does one of 2^31 - 1 rows.
+    The rows behind the bound are allocated."""
+    max_len, cap = 1000, 1152
+    q = oracle.normal(8100, (n_seq, nh * hd))
+    k, v = oracle.normal(8101, (n_seq * cap, nkv * hd)), oracle.normal(8102, (n_seq * cap, nkv * hd))
+    lens = np.resize(np.array([max_len + 1, max_len, 3, 2**31 - 1, 0, max_len - 1], np.int32), n_seq)
+    offs = np.arange(n_seq, dtype=np.int64) * cap
+    dq, dk, dv, do, dl = (ctx.upload(x) for x in (q, k, v, offs, lens))
+    dout = ctx.empty((n_seq, nh * hd))
+    dout.fill_bytes(0x3F)
+    if noalloc:
+        rc = ctx.lib.tmac_attention_decode_ragged_noalloc(ctx.handle, None, dq.ptr, dk.ptr, dv.ptr, do.ptr, dl.ptr,
+                                                          dout.ptr, n_seq, nh, nkv, hd, max_len, 0)
+        assert rc == tmac_attn.TMAC_OK
+    else:
+        ctx.decode_ragged(dq, dk, dv, do, dl, dout, n_seq, nh, nkv, hd, max_len)
+    got = dout.numpy()
+    assert ctx.check_device_error() == tmac_attn.TMAC_ERR_DEVICE_FAULT
+    for s in range(n_seq):
+        if lens[s] > max_len:
+            assert np.all(np.isnan(got[s])), f"sequence {s} of {lens[s]} rows"
+        elif lens[s] == 0:
+            assert np.all(got[s] == 0)
+        else:
+            ref = oracle.attention_ragged(q[s:s + 1], k, v, offs[s:s + 1], lens[s:s + 1], nh, nkv, hd, n_threads=8)
+            assert_close(got[s:s + 1], ref, f"sequence {s} of {lens[s]} rows")
+    for d in (dq, dk, dv, do, dl, dout):
+        d.free()

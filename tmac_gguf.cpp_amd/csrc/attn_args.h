@@ -80,10 +80,9 @@ struct DecodeArgs {
     const int32_t* positions;    // paged layer mode: [n_seq] position of each sequence's new token
     int max_pages;
     int n_pages;                 // pages in each pool
-    // stream-K ragged decode: per sequence (first workspace slot, slots used),
-    // and the launch's max_len (longer sequences give NaN and error bit 1)
+    // stream-K ragged decode: per sequence (first workspace slot, slots used)
     int32_t* seg_meta;
-    int sk_max_len;
+    int max_len;             // rows a sequence may have; longer ones give NaN and error bit 1
     // any-shape kernel (shapes without a compiled kernel): runtime kv heads and head_dim
     int n_kv_head;
     int head_dim;

@@ -674,6 +674,11 @@ __device__ __forceinline__ bool seq_geometry(const DecodeArgs& a, int seq, int& 
     return true;
 }
 
+// Splits that a sequence of n_pos rows (1 .. max_len) uses, at most n_splits.
+// A longer sequence is told by its length: max_len need not be a multiple of
+// split_len, and the rows past it may lie past the sequence's block table.
+__device__ __forceinline__ int active_splits(const DecodeArgs& a, int n_pos) { return (n_pos - 1) / a.split_len + 1; }
+
 // Flat unit grid (ragged and paged modes): unit index -> (sequence, split).
 // Sequence s with L_s = lengths[s] + add rows owns
 // clamp(ceil(L_s / split_len), 1, n_splits) consecutive units (a length above
@@ -834,8 +839,8 @@ __device__ __forceinline__ void decode_body(const DecodeArgs& a) {
             for (int i = threadIdx.x; i < KVS * GW * kHeadDim; i += NW * 64) out_heads[i] = 0.f;
         return;
     }
-    const int n_act = (n_pos + a.split_len - 1) / a.split_len;
-    if (n_act > a.n_splits) {  // length above the max_len the grid was sized for
+    const int n_act = active_splits(a, n_pos);
+    if (n_pos > a.max_len) {
         if (split == 0) {
             for (int i = threadIdx.x; i < KVS * GW * kHeadDim; i += NW * 64) out_heads[i] = __builtin_nanf("");
             if (threadIdx.x == 0) atomicOr(a.err, 2);
@@ -960,14 +965,14 @@ __device__ __forceinline__ bool sk_locate(const DecodeArgs& a, int64_t& S, int64
 #pragma unroll
     for (int r = 0; r < kKeep; ++r) {
         const int sq = r * NT + (int)threadIdx.x;
-        kept[r] = sq < a.n_seq ? sk_rows(sk_len<LAYER>(a, sq), a.sk_max_len) : 0;
+        kept[r] = sq < a.n_seq ? sk_rows(sk_len<LAYER>(a, sq), a.max_len) : 0;
     }
     int64_t mine = 0;
 #pragma unroll
     for (int r = 0; r < kKeep; ++r) mine += kept[r];
 #pragma unroll 8
     for (int sq = (int)threadIdx.x + kKeep * NT; sq < a.n_seq; sq += NT)
-        mine += sk_rows(sk_len<LAYER>(a, sq), a.sk_max_len);
+        mine += sk_rows(sk_len<LAYER>(a, sq), a.max_len);
 #pragma unroll
     for (int mask = 1; mask < 64; mask <<= 1) mine += __shfl_xor(mine, mask);
     if (lane == 0) s_wsum[wave] = mine;
@@ -995,7 +1000,7 @@ __device__ __forceinline__ bool sk_locate(const DecodeArgs& a, int64_t& S, int64
 #pragma unroll
             for (int j = 0; j < kKeep; ++j) rows = j == r ? kept[j] : rows;
         } else {
-            rows = sq < a.n_seq ? sk_rows(sk_len<LAYER>(a, sq), a.sk_max_len) : 0;
+            rows = sq < a.n_seq ? sk_rows(sk_len<LAYER>(a, sq), a.max_len) : 0;
         }
         int64_t incl = rows;
 #pragma unroll
@@ -1034,7 +1039,7 @@ __device__ __forceinline__ bool sk_seek(const DecodeArgs& a, int64_t lo, int64_t
     for (; s < a.n_seq && P < hi; ++s) {
         s = __builtin_amdgcn_readfirstlane(s);
         len = __builtin_amdgcn_readfirstlane(sk_len<LAYER>(a, s));
-        const int64_t rows = sk_rows(len, a.sk_max_len);
+        const int64_t rows = sk_rows(len, a.max_len);
         if (rows > 0 && lo - P < (int64_t)len) return true;  // lo - P < len: a row of s lies in [lo, hi)
         P += rows;
     }
@@ -1129,7 +1134,7 @@ __device__ __forceinline__ void decode_sk_body(const DecodeArgs& a) {
         if (PAGED && bad && lane == 0) atomicOr(a.err, 4);
         const bool direct = sk_record(a, s, P, len, S, last_u);
         int s2 = s + 1, len2 = 0;
-        int64_t P2 = P + sk_rows(len, a.sk_max_len);
+        int64_t P2 = P + sk_rows(len, a.max_len);
         const bool more = sk_seek<LAYER>(a, lo, hi, s2, P2, len2);
         if (more) load_q(q, s2);
         float* ws_slot = direct ? nullptr : a.ws + (size_t)(u + s) * NH * kPartialStride;
@@ -1626,9 +1631,9 @@ __device__ __forceinline__ void combine_body(const DecodeArgs& a) {
     int n_pos, pos;
     size_t base;
     if (!seq_geometry<MODE>(a, seq, n_pos, pos, base)) return;
-    if (n_pos <= 0) return;
-    const int n_act = (n_pos + a.split_len - 1) / a.split_len;
-    if (n_act <= 1 || n_act > a.n_splits) return;
+    if (n_pos <= 0 || n_pos > a.max_len) return;
+    const int n_act = active_splits(a, n_pos);
+    if (n_act <= 1) return;
     a.out[((size_t)seq * NH + h) * kHeadDim + d] = merge_splits<SP>(ws, n_act, d, &first);
 }
 
@@ -1657,7 +1662,7 @@ __device__ __forceinline__ void combine_sk_body(const DecodeArgs& a) {
         *o = 0.f;
         return;
     }
-    if (len > a.sk_max_len) {
+    if (len > a.max_len) {
         *o = __builtin_nanf("");
         if (h == 0 && d == 0) atomicOr(a.err, 2);
         return;
@@ -1992,14 +1997,14 @@ __device__ __forceinline__ void anyg_body(const DecodeArgs& a) {
     n_pos = __builtin_amdgcn_readfirstlane(n_pos);
     pos = __builtin_amdgcn_readfirstlane(pos);
     float* out = a.out + ((size_t)seq * a.n_head + head0) * hd;
-    const int n_act = (n_pos + a.split_len - 1) / a.split_len;
-    if (n_pos <= 0 || n_act > a.n_splits) {  // no rows: zeros; longer than the max_len the launch was sized for: NaN
+    if (n_pos <= 0 || n_pos > a.max_len) {  // no rows: zeros; longer than max_len: NaN
         if (split == 0) {
             for (int i = threadIdx.x; i < n_g * hd; i += NW * 64) out[i] = n_pos <= 0 ? 0.f : __builtin_nanf("");
             if (n_pos > 0 && threadIdx.x == 0) atomicOr(a.err, 2);
         }
         return;
     }
+    const int n_act = active_splits(a, n_pos);
     if (split >= n_act) return;
     const int mem_rows = MODE == kLayer ? pos : n_pos;  // layer mode: row pos comes from registers
     const int r0 = split * a.split_len;
@@ -2194,9 +2199,9 @@ __device__ __forceinline__ void any_combine_body(const DecodeArgs& a) {
     const int h = blockIdx.x, seq = blockIdx.y, hd = a.head_dim, d = min((int)threadIdx.x, hd - 1);
     int n_pos, pos;
     size_t base;
-    if (!seq_geometry<MODE>(a, seq, n_pos, pos, base) || n_pos <= 0) return;
-    const int n_act = (n_pos + a.split_len - 1) / a.split_len;
-    if (n_act <= 1 || n_act > a.n_splits) return;
+    if (!seq_geometry<MODE>(a, seq, n_pos, pos, base) || n_pos <= 0 || n_pos > a.max_len) return;
+    const int n_act = active_splits(a, n_pos);
+    if (n_act <= 1) return;
     const size_t SP = (size_t)a.n_head * (hd + 2);  // floats between splits
     const float* ws = a.ws + (size_t)seq * a.n_splits * SP + (size_t)h * (hd + 2);
     float M = kNegInf, L = 0.f, A = 0.f;
@@ -3670,8 +3675,8 @@ __device__ __forceinline__ void mdecode_body(const DecodeArgs& a) {
             for (int i = threadIdx.x; i < NH * kHeadDim; i += NW * 64) out_heads[i] = 0.f;
         return;
     }
-    const int n_act = (n_pos + a.split_len - 1) / a.split_len;
-    if (n_act > a.n_splits) {
+    const int n_act = active_splits(a, n_pos);
+    if (n_pos > a.max_len) {
         if (split == 0) {
             for (int i = threadIdx.x; i < NH * kHeadDim; i += NW * 64) out_heads[i] = __builtin_nanf("");
             if (threadIdx.x == 0) atomicOr(a.err, 2);
@@ -3704,7 +3709,7 @@ __device__ __forceinline__ void mdecode_sk_body(const DecodeArgs& a) {
         mdecode_segment<T, G, KV, PAGED ? kPaged : kRagged>(a, s, 0, 1, 0, PAGED ? 0 : (size_t)a.offsets[s],
                                                             (int)r0, (int)(r1 - r0),
                                                             a.out + (size_t)s * NH * kHeadDim, ws_slot);
-        P += sk_rows(len, a.sk_max_len);
+        P += sk_rows(len, a.max_len);
     }
 }
 

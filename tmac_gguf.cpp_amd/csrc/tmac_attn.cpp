@@ -599,6 +599,7 @@ int run_decode(tmac_context* ctx, hipStream_t stream, const Kernels& k, DecodeAr
     a.rot_mul = (int)ctx->opt_rot_mul;
     a.blocked = (int)ctx->opt_blocked;
     a.err = ctx->err;
+    a.max_len = grid_rows;
     if (n_seq > 65535) return fail(ctx, TMAC_ERR_INVALID_ARG, "n_seq exceeds 65535");
     if (k.any) return run_decode_any(ctx, stream, k, a, n_seq, grid_rows, n_kv_head);
     const bool unit_grid = a.lengths || a.positions;  // ragged and paged modes
@@ -717,7 +718,7 @@ int run_decode_sk(tmac_context* ctx, hipStream_t stream, hipFunction_t sk, unsig
     a.rot_mul = (int)ctx->opt_rot_mul;
     a.blocked = (int)ctx->opt_blocked;
     a.err = ctx->err;
-    a.sk_max_len = max_len;
+    a.max_len = max_len;
     if (n_seq > 65535) return fail(ctx, TMAC_ERR_INVALID_ARG, "n_seq exceeds 65535");
     if (max_len > INT_MAX - kPageRows) return fail(ctx, TMAC_ERR_INVALID_ARG, "stream-K decode: max_len too large");
     // One workgroup per CU; two when the sequences outnumber the CUs (more
