@@ -266,3 +266,44 @@ def test_any_shape_length_bound_is_exact(ctx, nh, nkv, hd, n_seq, noalloc):
             assert_close(got[s:s + 1], ref, f"sequence {s} of {lens[s]} rows")
     for d in (dq, dk, dv, do, dl, dout):
         d.free()
+
+
+@pytest.mark.parametrize("nh,nkv,hd", [(14, 2, 128), (5, 5, 256), (6, 3, 64), (9, 3, 66)])
+def test_any_shape_infinite_rows(ctx, nh, nkv, hd):
+    """An infinity in V reaches the output as an infinity, not as a NaN of a masked slot (0 * inf),
+    also in the last row of a partial step and in the layer step's new row; a key that scores -inf
+    weighs nothing, also where it is the only row of the last split (lengths 161, 321 and 801 of
+    max_len 1,000, whose splits hold 160 rows at 14 / 2 heads)."""
+    max_len, lens = 1000, np.array([161, 321, 801, 2, 999], np.int32)
+    n_seq = lens.size
+    offs = np.arange(n_seq, dtype=np.int64) * max_len
+    q = np.abs(oracle.normal(8200, (n_seq, nh * hd))) + 0.1  # every head scores a key of -inf in dim 1 as -inf
+    k, v = oracle.normal(8201, (n_seq * max_len, nkv * hd)), oracle.normal(8202, (n_seq * max_len, nkv * hd))
+    last = offs + lens - 1
+    ki, vi = k.copy(), v.copy()
+    ki[last, 1::hd] = -np.inf
+    vi[last, 0::hd] = np.inf
+    dq, dk, dv, dki, dvi, do, dl = (ctx.upload(x) for x in (q, k, v, ki, vi, offs, lens))
+    dout = ctx.empty((n_seq, nh * hd))
+    ctx.decode_ragged(dq, dki, dv, do, dl, dout, n_seq, nh, nkv, hd, max_len)
+    ref = oracle.attention_ragged(q, k, v, offs, lens - 1, nh, nkv, hd, n_threads=8)  # without the last row
+    assert_close(dout.numpy(), ref, f"key of score -inf, {nh}/{nkv}/{hd}")
+    ctx.decode_ragged(dq, dk, dvi, do, dl, dout, n_seq, nh, nkv, hd, max_len)
+    got = dout.numpy()
+    ref = oracle.attention_ragged(q, k, v, offs, lens, nh, nkv, hd, n_threads=8)
+    first = np.arange(nh * hd) % hd == 0
+    assert np.all(got[:, first] == np.inf)
+    assert_close(got[:, ~first], ref[:, ~first], f"infinity in V, {nh}/{nkv}/{hd}")
+    pos = 40
+    kn, vn = oracle.normal(8203, nkv * hd), oracle.normal(8204, nkv * hd)
+    vn[0::hd] = np.inf
+    dkn, dvn = ctx.upload(kn), ctx.upload(vn)
+    ctx.layer_attention(dq, dkn, dvn, dk, dv, dout, nh, nkv, hd, pos, max_len, 1e6)
+    got = dout.numpy()[0]
+    vn[0::hd] = 0
+    ref, _, _ = oracle.layer_step(q[0], kn, vn, k[:max_len], v[:max_len], nh, nkv, hd, pos, 1e6)
+    assert np.all(got[first] == np.inf)
+    assert_close(got[~first], ref[~first], f"infinity in v_new, {nh}/{nkv}/{hd}")
+    for d in (dq, dk, dv, dki, dvi, do, dl, dout, dkn, dvn):
+        d.free()
+    assert ctx.check_device_error() == 0

@@ -1953,6 +1953,9 @@ __device__ __forceinline__ void any_body(const DecodeArgs& a) {
 // ([sequence][split][head][head_dim + 2]: acc, m, l) are merged by a second
 // launch.  Lanes whose chunk lies past head_dim load chunk 0 and score 0.
 constexpr int kAnyDepth = 3;
+// Running max before any score: the lowest finite value, so that a row of score -inf (an infinity in k) has the
+// weight exp2(-inf - kNoMax) = 0 also where it is all that a wave or a split holds.
+constexpr float kNoMax = -__FLT_MAX__;
 
 template <int L>
 __device__ __forceinline__ float lanes_sum(float x) {  // over L consecutive lanes
@@ -2035,7 +2038,7 @@ __device__ __forceinline__ void anyg_body(const DecodeArgs& a) {
     float m[GT], l[GT], acc[GT][8];
 #pragma unroll
     for (int g = 0; g < GT; ++g) {
-        m[g] = kNegInf;
+        m[g] = kNoMax;
         l[g] = 0.f;
 #pragma unroll
         for (int t = 0; t < 8; ++t) acc[g][t] = 0.f;
@@ -2063,7 +2066,7 @@ __device__ __forceinline__ void anyg_body(const DecodeArgs& a) {
 #pragma unroll
             for (int g = 0; g < GT; ++g) {
                 const float mn = fmaxf(m[g], xor_max<1>(s[g]));
-                const float alpha = (m[g] == kNegInf) ? 0.f : fast_exp2(m[g] - mn);
+                const float alpha = fast_exp2(m[g] - mn);
                 l[g] *= alpha;
 #pragma unroll
                 for (int t = 0; t < 8; ++t) acc[g][t] *= alpha;
@@ -2075,7 +2078,7 @@ __device__ __forceinline__ void anyg_body(const DecodeArgs& a) {
             const float e = fast_exp2(s[g] - m[g]);
             l[g] += e;
 #pragma unroll
-            for (int t = 0; t < 8; ++t) acc[g][t] = fmaf(e, vf[t], acc[g][t]);
+            for (int t = 0; t < 8; ++t) acc[g][t] = fmaf(e, !MASKED || valid ? vf[t] : 0.f, acc[g][t]);
         }
     };
 
@@ -2173,8 +2176,7 @@ __device__ __forceinline__ void anyg_body(const DecodeArgs& a) {
         float L = 0.f, A = 0.f;
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
-            const float mw = s_m[w][g];
-            const float sc = (mw == kNegInf) ? 0.f : fast_exp2(mw - M);
+            const float sc = fast_exp2(s_m[w][g] - M);
             L = fmaf(s_l[w][g], sc, L);
             A = fmaf(s_acc[w][g][d], sc, A);
         }
@@ -2217,17 +2219,16 @@ __device__ __forceinline__ void any_combine_body(const DecodeArgs& a) {
         float nm = M;
 #pragma unroll
         for (int j = 0; j < kAnyMerge; ++j) {
-            m[j] = u0 + j < n_act ? m[j] : kNegInf;
-            nm = fmaxf(nm, m[j]);  // finite: every split holds a row
+            nm = fmaxf(nm, m[j]);  // at least kNoMax
         }
         const float sc = (M == kNegInf) ? 0.f : fast_exp2(M - nm);
         L *= sc;
         A *= sc;
 #pragma unroll
-        for (int j = 0; j < kAnyMerge; ++j) {
-            const float e = (m[j] == kNegInf) ? 0.f : fast_exp2(m[j] - nm);
-            L = fmaf(l[j], e, L);
-            A = fmaf(x[j], e, A);
+        for (int j = 0; j < kAnyMerge; ++j) {  // (repeats of the last split stay out: 0 * inf is NaN)
+            const float e = fast_exp2(m[j] - nm);
+            L = u0 + j < n_act ? fmaf(l[j], e, L) : L;
+            A = u0 + j < n_act ? fmaf(x[j], e, A) : A;
         }
         M = nm;
     }
