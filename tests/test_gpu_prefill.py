@@ -410,3 +410,24 @@ def test_prefill_key_runs(ctx, n_seq, n_q, prefix, n_head, n_kv):
     for d in (dq, dk, dv, tiles, out):
         d.free()
     assert ctx.check_device_error() == 0
+
+
+@pytest.mark.parametrize("n_q,prefix", [(16, 300), (17, 4000), (1, 1023), (33, 2100)])
+def test_prefill_infinity_in_v(ctx, n_q, prefix):
+    """An infinity in V that every query sees reaches the output as an infinity, with whole blocks
+    (prefix 300) and with key runs, whose merge repeats the last run in the slots it does not fill:
+    in the first row, and in the last row before the chunk (the last run of the first queries).
+    Their keys are scaled down: a row that scores the maximum has the weight 1, whose second bf16
+    part is 0, and 0 * inf is NaN in every prefill."""
+    n_head, n_kv = 14, 2
+    cap = prefix + n_q
+    q, k, v = (bf16_round(a) for a in make(950 + n_q, 1, n_q, prefix, cap, n_head, n_kv))
+    k.reshape(cap, n_kv * HD)[[0, prefix - 1]] *= 0.25
+    ref = oracle.prefill(q, k, v, 1, n_q, prefix, cap, n_head, n_kv, HD, n_threads=8)
+    first = np.arange(ref.size // n_q) % HD == 0
+    for row in (0, prefix - 1):
+        vi = v.copy()
+        vi.reshape(cap, n_kv * HD)[row, 0::HD] = np.inf
+        got = run(ctx, q, k, vi, 1, n_q, prefix, cap, n_head, n_kv).reshape(n_q, -1)
+        assert np.all(got[:, first] == np.inf), f"row {row}"
+        assert_close(got[:, ~first], ref.reshape(n_q, -1)[:, ~first], f"row {row}, the other dims")

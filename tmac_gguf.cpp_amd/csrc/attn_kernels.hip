@@ -2850,7 +2850,6 @@ __device__ __forceinline__ void prefill_combine_body(const PrefillArgs& a) {
         float nm = M;
 #pragma unroll
         for (int j = 0; j < kMergeRuns; ++j) {
-            m[j] = u0 + j < n_act ? m[j] : kNegInf;
             nm = fmaxf(nm, m[j]);
         }
         // (nm is finite: every column sees key 0, which is in the first run)
@@ -2861,9 +2860,10 @@ __device__ __forceinline__ void prefill_combine_body(const PrefillArgs& a) {
 #pragma unroll
         for (int j = 0; j < kMergeRuns; ++j) {
             const float w = (m[j] == kNegInf) ? 0.f : fast_exp2(m[j] - nm);
-            L = fmaf(l[j], w, L);
+            const bool in = u0 + j < n_act;  // (repeats of the last run stay out: 0 * inf is NaN)
+            L = in ? fmaf(l[j], w, L) : L;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) A[i] = fmaf(x[j][i], w, A[i]);
+            for (int i = 0; i < 4; ++i) A[i] = in ? fmaf(x[j][i], w, A[i]) : A[i];
         }
         M = nm;
     }
