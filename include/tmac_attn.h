@@ -230,8 +230,8 @@ int tmac_attention_decode_ragged(tmac_context* ctx, tmac_stream stream, const fl
  * process ends, instead of the context's growable workspace, and the call never calls hipMalloc or
  * hipFree.  A call whose schedule needs more than TMAC_SCRATCH_BYTES of partials launches nothing and
  * returns TMAC_ERR_CAPACITY (at 14 query heads: stream-K batches up to about 4,000 sequences, unit-grid
- * batches up to n_seq * splits = 4,500); a shape without compiled kernels then keeps its rows
- * unsplit instead.  Every call on one GPU shares that GPU's array (all contexts
+ * batches up to n_seq * splits = 4,500; the splits of a shape without compiled kernels always
+ * fit).  Every call on one GPU shares that GPU's array (all contexts
  * and streams): calls that overlap on one GPU race.  No part of it needs to start at zero. */
 #define TMAC_SCRATCH_BYTES (16u << 20)
 int tmac_attention_decode_ragged_noalloc(tmac_context* ctx, tmac_stream stream, const float* q,
@@ -349,8 +349,8 @@ int tmac_layer_attention_paged(tmac_context* ctx, tmac_stream stream, int kv_dty
  * up to 256 rows), which grows on demand; a call that needs it to grow while
  * the stream is capturing returns TMAC_ERR_CAPTURE, so run the largest shape
  * once before capture.  Few queries after many rows: the rows are cut into runs
- * and a third launch merges their partials, also in the workspace (where that
- * cannot grow for them, the rows stay whole: the same results up to rounding). */
+ * and a third launch merges their partials, in a buffer the context holds from
+ * tmac_init on. */
 int tmac_attention_prefill(tmac_context* ctx, tmac_stream stream, const float* q, const float* k_cache,
                            const float* v_cache, float* out, int n_seq, int n_q, int prefix_len,
                            int64_t seq_stride, int n_head, int n_kv_head, int head_dim);
@@ -383,8 +383,7 @@ int tmac_attention_prefill_paged(tmac_context* ctx, tmac_stream stream, int kv_d
  *   tmac_attention_prefill_tiles: the attention of tmac_attention_prefill over the tiles,
  *     which must hold rows 0 .. prefix_len + n_q - 1 (prefix_len + n_q <= capacity).
  * pack_rows(0, prefix_len + n_q) then attention_prefill_tiles gives the outputs of
- * tmac_attention_prefill bit for bit (the same kernels on the same tiles; under capture,
- * if the workspace has held the same shape's runs before). */
+ * tmac_attention_prefill bit for bit (the same kernels on the same tiles). */
 size_t tmac_prefill_tiles_bytes(int n_seq, int n_kv_head, int capacity);
 int tmac_prefill_pack_rows(tmac_context* ctx, tmac_stream stream, int kv_dtype, const void* k_cache,
                            const void* v_cache, int64_t seq_stride, void* tiles, int capacity, int n_seq,

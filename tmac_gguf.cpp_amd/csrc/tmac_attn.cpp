@@ -62,6 +62,11 @@ using tmac::kPageRows;
 namespace {
 
 constexpr int kHeadMaxRows = 1024;  // automatic choice: head kernel up to this many rows
+// The context's partials buffer, in prefill slots (one unit's kMaxGroup heads) per CU.  Key runs: at most n_cu units
+// over blocks of which the longest has the most runs; the slots, blocks times its runs, come to 492 at most on 256
+// CUs (every count of blocks and prefix tried).  Any-shape splits: fewer than 4 workgroups of 8 heads per CU, which
+// at 258 floats a head is less than half of this.
+constexpr int kPartSlotsPerCu = 2, kMaxGroup = 8;
 // (G = n_head / n_kv_head, KV = n_kv_head) pairs compiled into the code object.
 constexpr int kShapes[][2] = {{7, 2}, {1, 1}, {1, 2}, {2, 2}, {4, 2}, {4, 4}, {8, 1}};
 enum { kModeUniform = 0, kModeRagged = 1, kModeLayer = 2 };
@@ -132,6 +137,12 @@ struct tmac_context {
     hipFunction_t k_gemv_q8 = nullptr, k_gemv_q5 = nullptr, k_kq[2][2] = {};
     float* ws = nullptr;
     size_t ws_floats = 0;
+    // Partials of the any-shape splits and of the prefill key runs: as large as
+    // any call can need (kPartSlotsPerCu), allocated at init and never replaced,
+    // so that these schedules depend on the shape alone, not on whether the
+    // workspace has grown, may grow (capture) or moves under a captured graph.
+    float* part = nullptr;
+    size_t part_floats = 0;
     int* err = nullptr;
     // The library's own copies and fills (tables, tags, the error word) go on
     // this non-blocking stream and wait for it alone: on this runtime a
@@ -556,7 +567,8 @@ const float kQScale = (float)(1.4426950408889634 / 8.0);  // log2(e) / sqrt(64)
 // the rows are split until the workgroups reach kAnyTargetPerCu per CU, into
 // runs of at least kAnyMinRows rows, and batches that still leave half of the
 // CUs idle serve fewer heads per workgroup (each then reads the rows through
-// L2).  Without room for the splits' partials the rows stay whole.
+// L2).  The partials fit the context's buffer, and the fixed scratch array of
+// the no-allocation entry point: fewer than 4 units of 8 heads per CU.
 constexpr int kAnyTargetPerCu = 2, kAnyMinRows = 128;
 int run_decode_any(tmac_context* ctx, hipStream_t stream, const Kernels& k, DecodeArgs& a, int n_seq, int grid_rows,
                    int n_kv_head) {
@@ -577,10 +589,10 @@ int run_decode_any(tmac_context* ctx, hipStream_t stream, const Kernels& k, Deco
         const int64_t len = (((int64_t)grid_rows + want - 1) / want + 31) / 32 * 32;
         const int n_splits = (int)((grid_rows + len - 1) / len);
         const size_t floats = (size_t)n_seq * n_splits * a.n_head * (a.head_dim + 2);
-        if (n_splits > 1 && ensure_workspace(ctx, stream, floats) == TMAC_OK) {
+        if (n_splits > 1 && floats <= (ctx->fixed_ws ? ctx->fixed_floats : ctx->part_floats)) {
             a.split_len = (int)len;
             a.n_splits = n_splits;
-            a.ws = workspace(ctx);
+            a.ws = ctx->fixed_ws ? ctx->fixed_ws : ctx->part;
         }
     }
     while (gt > 0 && (int64_t)n_seq * n_kv_head * tiles() * a.n_splits * 2 <= ctx->n_cu) gt--;
@@ -781,6 +793,7 @@ int tmac_init(tmac_context** out, int device) {
     auto bail = [&](int rc) {
         if (ctx->aux) (void)hipStreamSynchronize(ctx->aux);
         if (ctx->ws) (void)hipFree(ctx->ws);
+        if (ctx->part) (void)hipFree(ctx->part);
         if (ctx->err) (void)hipFree(ctx->err);
         if (ctx->pos_slot_pool) (void)hipFree(ctx->pos_slot_pool);
         if (ctx->aux) (void)hipStreamDestroy(ctx->aux);
@@ -965,6 +978,9 @@ int tmac_init(tmac_context** out, int device) {
         return bail(hip_fail(ctx, e, "hipMemsetAsync"));  // every tag -1: no slot holds a row yet
     int rc = ensure_workspace(ctx, nullptr, (size_t)1 << 20);
     if (rc) return bail(rc);
+    ctx->part_floats = (size_t)kPartSlotsPerCu * ctx->n_cu * kMaxGroup * tmac::kPrefillPartFloats;
+    if ((e = hipMalloc(&ctx->part, ctx->part_floats * sizeof(float))) != hipSuccess)
+        return bail(hip_fail(ctx, e, "hipMalloc"));
     void* scratch = nullptr;
     if ((e = (hipError_t)tmac_scratch_setup(device, &scratch)) != hipSuccess)
         return bail(hip_fail(ctx, e, "hipGetSymbolAddress(scratch)"));
@@ -983,6 +999,7 @@ int tmac_shutdown(tmac_context* ctx) {
         if (ctx->aux) (void)hipStreamSynchronize(ctx->aux);
         for (auto& t : ctx->rope) (void)hipFree(t.dev);
         if (ctx->ws) (void)hipFree(ctx->ws);
+        if (ctx->part) (void)hipFree(ctx->part);
         for (void* p : ctx->retired) (void)hipFree(p);
         for (tmac_graph* g : ctx->graphs) g->owner = nullptr;  // graphs destroyed later touch no context
         if (ctx->err) (void)hipFree(ctx->err);
@@ -1341,13 +1358,12 @@ struct PrefillPlan {
     int split;        // stages per unit, 0: one unit per block
     int n_parts;      // units of the longest block
     int64_t n_blocks; // units of all (sequence, kv head) pairs
-    size_t floats;    // workspace for the partials
     int n_qblk;
 };
 
 static PrefillPlan whole_blocks(int n_sk, int n_q) {
     const int n_qblk = (n_q + kPrefillQueries - 1) / kPrefillQueries;
-    return PrefillPlan{0, 1, (int64_t)n_qblk * n_sk, 0, n_qblk};
+    return PrefillPlan{0, 1, (int64_t)n_qblk * n_sk, n_qblk};
 }
 
 static PrefillPlan prefill_plan(const tmac_context* ctx, int n_sk, int group, int n_q, int prefix_len) {
@@ -1359,14 +1375,16 @@ static PrefillPlan prefill_plan(const tmac_context* ctx, int n_sk, int group, in
         return (prefix_len + std::min((b + 1) * kPrefillQueries, n_q) - 1) / (kPrefillKeys * kPrefillStageTiles) + 1;
     };
     const int n_qblk = best.n_qblk, longest = stages(n_qblk - 1);
-    for (int split = 1; split + kMergeStages < longest; split++) {
+    int64_t total = 0;
+    for (int b = 0; b < n_qblk; b++) total += (int64_t)n_sk * stages(b);
+    for (int split = (int)std::max<int64_t>(1, total / ctx->n_cu); split + kMergeStages < longest; split++) {
         int64_t units = 0;
         for (int b = 0; b < n_qblk; b++) units += (stages(b) + split - 1) / split;
         units *= n_sk;
         if (units > ctx->n_cu) continue;
         const int n_parts = (longest + split - 1) / split;
-        return PrefillPlan{split, n_parts, units, (size_t)n_sk * n_qblk * n_parts * group * tmac::kPrefillPartFloats,
-                           n_qblk};
+        const size_t floats = (size_t)n_sk * n_qblk * n_parts * group * tmac::kPrefillPartFloats;
+        if (floats <= ctx->part_floats) return PrefillPlan{split, n_parts, units, n_qblk};
     }
     return best;
 }
@@ -1417,17 +1435,12 @@ static int prefill_impl(tmac_context* ctx, tmac_stream stream, int dt, const flo
     const int64_t pack_blocks = (int64_t)n_tp * n_kv_head * n_seq;
     if (pack_blocks > INT_MAX) return fail(ctx, TMAC_ERR_INVALID_ARG, "prefill: too many cache tiles");
     const size_t pack_floats = (size_t)pack_blocks * kPrefillTileElems * sizeof(uint16_t) / sizeof(float);
-    PrefillPlan plan = prefill_plan(ctx, n_seq * n_kv_head, n_head / n_kv_head, n_q, prefix_len);
-    rc = ensure_workspace(ctx, (hipStream_t)stream, pack_floats + plan.floats);
-    if (rc && plan.split) {  // no room for the partials (a capturing stream): one unit per block
-        plan = whole_blocks(n_seq * n_kv_head, n_q);
-        rc = ensure_workspace(ctx, (hipStream_t)stream, pack_floats);
-    }
-    if (rc) return rc;
+    const PrefillPlan plan = prefill_plan(ctx, n_seq * n_kv_head, n_head / n_kv_head, n_q, prefix_len);
+    if ((rc = ensure_workspace(ctx, (hipStream_t)stream, pack_floats))) return rc;
     PrefillArgs a{q, static_cast<const float*>(k_cache), static_cast<const float*>(v_cache), out, seq_stride, n_q,
                   prefix_len, plan.n_qblk, kQScale, reinterpret_cast<uint16_t*>(workspace(ctx)), n_tp, n_rows, 0,
                   n_tp, block_table, max_pages, n_pages, ctx->err, 0, n_seq * n_kv_head, plan.split, plan.n_parts,
-                  workspace(ctx) + pack_floats};
+                  ctx->part};
     if ((rc = launch(ctx, ctx->prefill_pack[block_table ? 1 : 0][dt].at(n_kv_head), (unsigned)pack_blocks, 1, 256,
                      (hipStream_t)stream, &a)))
         return rc;
@@ -1525,13 +1538,11 @@ int tmac_attention_prefill_tiles(tmac_context* ctx, tmac_stream stream, const fl
     if (!ctx->prefill.count({n_head / n_kv_head, n_kv_head}))
         return fail(ctx, TMAC_ERR_UNSUPPORTED, "prefill_tiles: unsupported group");
     if ((rc = set_device(ctx))) return rc;
-    PrefillPlan plan = prefill_plan(ctx, n_seq * n_kv_head, n_head / n_kv_head, n_q, prefix_len);
-    if (plan.split && ensure_workspace(ctx, (hipStream_t)stream, plan.floats) != TMAC_OK)
-        plan = whole_blocks(n_seq * n_kv_head, n_q);  // no room for the partials: one unit per block, no workspace
+    const PrefillPlan plan = prefill_plan(ctx, n_seq * n_kv_head, n_head / n_kv_head, n_q, prefix_len);
     PrefillArgs a{q, nullptr, nullptr, out, 0, n_q, prefix_len, plan.n_qblk, kQScale,
                   static_cast<uint16_t*>(const_cast<void*>(tiles)), prefill_tiles_per_head(capacity),
                   prefix_len + n_q, 0, 0, nullptr, 0, 0, ctx->err, 0, n_seq * n_kv_head, plan.split, plan.n_parts,
-                  workspace(ctx)};
+                  ctx->part};
     return launch_prefill(ctx, (hipStream_t)stream, n_head, n_kv_head, plan, a);
 }
 
