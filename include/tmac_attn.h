@@ -395,7 +395,9 @@ int tmac_attention_prefill_tiles(tmac_context* ctx, tmac_stream stream, const fl
 /* ---- tuning / introspection ---- */
 enum tmac_option {
     TMAC_OPT_SPLIT_LEN = 1,     /* group kernel: rows per workgroup; 0 = automatic (default) */
-    TMAC_OPT_TARGET_GROUPS = 2, /* workgroups the automatic split aims for; 0 = one per CU */
+    TMAC_OPT_TARGET_GROUPS = 2, /* workgroups the automatic split aims for; 0 (default) = one per CU, or two where
+                                   ragged and paged decode of bf16 / fp16 caches is given total_rows and gains from
+                                   more parts to even out the lengths */
     TMAC_OPT_KERNEL = 3,        /* a tmac_kernel_choice */
     TMAC_OPT_ROTATE = 4,        /* decode: workgroup w starts w*value steps into its rows (default 0) */
     TMAC_OPT_HEAD_WAVES = 5,    /* head kernel workgroup size in waves: 4, 8 or 16 (default 8) */

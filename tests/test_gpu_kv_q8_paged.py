@@ -854,3 +854,44 @@ def test_units_two_per_cu(ctx, dt, n_seq, max_len):
     for x in d + [dout]:
         x.free()
     assert ctx.check_device_error() == 0
+
+
+def ragged_bits(ctx, n_seq, max_len, lens, options):
+    """Bits of a hinted bf16 ragged decode (sequences share a pool of rows) under `options`."""
+    rng = np.random.default_rng(n_seq)
+    pool = 2 * max_len
+    offs = rng.integers(0, pool - max_len + 1, n_seq).astype(np.int64)
+    kv = [(rng.standard_normal((pool, 128), dtype=np.float32).view(np.uint32) >> 16).astype(np.uint16) for _ in range(2)]
+    d = [ctx.upload(x) for x in (rng.standard_normal((n_seq, 14 * 64), dtype=np.float32), *kv, offs, lens)]
+    dout = ctx.empty((n_seq, 14 * 64))
+    for option, value in options.items():
+        ctx.set_option(option, value)
+    try:
+        ctx.decode_ragged(*d, dout, n_seq, 14, 2, 64, max_len, total_rows=int(lens.sum()), kv_dtype=tmac_attn.TMAC_KV_BF16)
+        got = dout.numpy().view(np.uint32)
+    finally:
+        for option in options:
+            ctx.set_option(option, 0)
+    for x in d + [dout]:
+        x.free()
+    return got
+
+
+def one_unit_split(n_cu, n_seq, max_len, total):
+    """Rows a split holds where the splits aim at one unit per CU (steps of 16 rows over 4 waves)."""
+    whole = -(-max_len // 16) * 16
+    return whole if n_seq >= n_cu else min(-(-(-(-total // (n_cu - n_seq))) // 16) * 16, whole)
+
+
+@pytest.mark.parametrize("n_seq,max_len", [(193, 4096), (144, 3000), (300, 2000)])
+def test_target_groups_option_is_taken_as_given(ctx, n_seq, max_len):
+    """TMAC_OPT_TARGET_GROUPS = the CUs splits the hinted 16-bit decode for one workgroup per CU, not for two:
+    the bits of that split length, which differ from those of half of it."""
+    n_cu = ctx.device_info()[1]
+    lens = np.random.default_rng(n_seq).integers(1, max_len + 1, n_seq).astype(np.int32)
+    lens[0] = max_len
+    want = one_unit_split(n_cu, n_seq, max_len, int(lens.sum()))
+    got = ragged_bits(ctx, n_seq, max_len, lens, {tmac_attn.TMAC_OPT_TARGET_GROUPS: n_cu})
+    np.testing.assert_array_equal(got, ragged_bits(ctx, n_seq, max_len, lens, {tmac_attn.TMAC_OPT_SPLIT_LEN: want}))
+    assert np.any(got != ragged_bits(ctx, n_seq, max_len, lens, {tmac_attn.TMAC_OPT_SPLIT_LEN: want // 32 * 16}))
+    assert ctx.check_device_error() == 0

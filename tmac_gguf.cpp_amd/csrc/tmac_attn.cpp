@@ -361,7 +361,8 @@ void choose_split(const tmac_context* ctx, int waves, int n_seq, int n_pos, int 
     // The 4-wave MFMA decode (bf16 / fp16 caches) holds two workgroups on a CU.
     // With a sequence for every second or third CU or more, one unit per CU
     // leaves too few units to even out the lengths: two per CU, the longest
-    // sequence cut into equal parts.  Lengths U[1, L], bf16, us: 128 x 4096
+    // sequence cut into equal parts.  Not where TMAC_OPT_TARGET_GROUPS names
+    // the workgroups to aim for.  Lengths U[1, L], bf16, us: 128 x 4096
     // 32.1 -> 29.4, 193 x 4096 55.0 -> 44.5, 300 x 2000 45.9 -> 37.8; below
     // that line nothing gained (64 x 16384 56.7, 59.2), and the 8-wave Q8_0
     // kernel, one workgroup per CU, is mixed (193 x 4096 45.9 -> 39.1, 220 x
@@ -369,10 +370,12 @@ void choose_split(const tmac_context* ctx, int waves, int n_seq, int n_pos, int 
     // Lengths so unequal that this would take more than 3.5 slots per CU keep
     // the other rules, so the partials fit the workspace a context starts with.
     int64_t equal_parts = 0;
-    if (total_rows > 0 && two_per_cu && 8 * (int64_t)n_seq >= 3 * target_groups && 2 * target_groups > n_seq) {
-        const int64_t per = (total_rows + (2 * target_groups - n_seq) - 1) / (2 * target_groups - n_seq);
+    const int64_t n_cu = ctx->n_cu;
+    if (total_rows > 0 && two_per_cu && ctx->opt_target_groups == 0 && 8 * (int64_t)n_seq >= 3 * n_cu &&
+        2 * n_cu > n_seq) {
+        const int64_t per = (total_rows + (2 * n_cu - n_seq) - 1) / (2 * n_cu - n_seq);
         const int64_t parts = (n_pos + per - 1) / per;
-        if (2 * parts * n_seq <= 7 * target_groups) equal_parts = parts;
+        if (2 * parts * n_seq <= 7 * n_cu) equal_parts = parts;
     }
     if (ctx->opt_split_len > 0) {
         len = (int)(((ctx->opt_split_len + round - 1) / round) * round);
