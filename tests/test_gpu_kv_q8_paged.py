@@ -895,3 +895,27 @@ def test_target_groups_option_is_taken_as_given(ctx, n_seq, max_len):
     np.testing.assert_array_equal(got, ragged_bits(ctx, n_seq, max_len, lens, {tmac_attn.TMAC_OPT_SPLIT_LEN: want}))
     assert np.any(got != ragged_bits(ctx, n_seq, max_len, lens, {tmac_attn.TMAC_OPT_SPLIT_LEN: want // 32 * 16}))
     assert ctx.check_device_error() == 0
+
+
+@pytest.mark.parametrize("n_seq,max_len,lo,hi,parts", [
+    (193, 4096, 0, 1, 4), (100, 8192, 0, 1, 8), (300, 2000, 0, 1, 2),
+    (193, 4096, 0.9, 1, 0),      # rows of a like length
+    (193, 1000, 0, 1, 0),        # short parts
+    (250, 4096, 0.3, 0.8, 0),    # two parts at up to a sequence per CU
+    (270, 4096, 0, 1, 0)])       # up to 9 sequences per 8 CUs
+def test_two_units_per_cu_rule(ctx, n_seq, max_len, lo, hi, parts):
+    """The bits of a hinted bf16 decode are those of the split length the rule gives on 256 CUs: max_len cut
+    into `parts`, or (0) one unit per CU, and not those of the other one."""
+    n_cu = ctx.device_info()[1]
+    if n_cu != 256:
+        pytest.skip("the parts are those of 256 CUs")
+    f = np.random.default_rng(n_seq + 1).uniform(lo, hi, n_seq)
+    lens = np.maximum(1, (f * max_len).astype(np.int32))
+    lens[0] = max_len
+    one = one_unit_split(n_cu, n_seq, max_len, int(lens.sum()))
+    two = -(-(-(-max_len // (parts or 2))) // 16) * 16
+    want, other = (two, one) if parts else (one, two)
+    got = ragged_bits(ctx, n_seq, max_len, lens, {})
+    np.testing.assert_array_equal(got, ragged_bits(ctx, n_seq, max_len, lens, {tmac_attn.TMAC_OPT_SPLIT_LEN: want}))
+    assert np.any(got != ragged_bits(ctx, n_seq, max_len, lens, {tmac_attn.TMAC_OPT_SPLIT_LEN: other}))
+    assert ctx.check_device_error() == 0

@@ -359,23 +359,33 @@ void choose_split(const tmac_context* ctx, int waves, int n_seq, int n_pos, int 
     int len;
     const int64_t target_groups = ctx->opt_target_groups > 0 ? ctx->opt_target_groups : (int64_t)ctx->n_cu;
     // The 4-wave MFMA decode (bf16 / fp16 caches) holds two workgroups on a CU.
-    // With a sequence for every second or third CU or more, one unit per CU
-    // leaves too few units to even out the lengths: two per CU, the longest
-    // sequence cut into equal parts.  Not where TMAC_OPT_TARGET_GROUPS names
-    // the workgroups to aim for.  Lengths U[1, L], bf16, us: 128 x 4096
-    // 32.1 -> 29.4, 193 x 4096 55.0 -> 44.5, 300 x 2000 45.9 -> 37.8; below
-    // that line nothing gained (64 x 16384 56.7, 59.2), and the 8-wave Q8_0
-    // kernel, one workgroup per CU, is mixed (193 x 4096 45.9 -> 39.1, 220 x
-    // 3000 35.9 -> 37.7, 128 x 4096 31.2 -> 31.9) and keeps one unit per CU.
-    // Lengths so unequal that this would take more than 3.5 slots per CU keep
-    // the other rules, so the partials fit the workspace a context starts with.
+    // Where the lengths differ widely and one unit per CU is too few to even
+    // them out: two per CU, the longest sequence cut into equal parts.  Not
+    // where TMAC_OPT_TARGET_GROUPS names the workgroups to aim for.  The merge
+    // launch and shorter units cost more than that gives for rows of a like
+    // length (193 x 1000 equal rows 22.9 -> 27.3 us, 193 x 4096 63.0 -> 70.6),
+    // in short parts (256 x U[1, 300] 11.7 -> 17.0), and where whole sequences
+    // nearly fill the CUs: two parts each at up to a sequence per CU (240 x
+    // half of 4096, half of 512 rows 54.2 -> 63.1), and up to 9 sequences per
+    // 8 CUs.  So: a mean of at most 9/16 of max_len, parts of 768 rows or more,
+    // three parts or more than 9/8 sequences per CU.  Over 1280 batches (1, 8,
+    // 14 and 16 query heads, 96 to 511 sequences, max_len 300 to 8192, four
+    // kinds of lengths) that takes 264, up to 37 % faster, none more than 2 %
+    // slower than one unit per CU: U[1, L] 193 x 4096 50.1 -> 41.1, 160 x 4096
+    // 45.7 -> 35.2, 300 x 2000 46.1 -> 38.1.  The 8-wave Q8_0 kernel, one
+    // workgroup per CU, is mixed (193 x 4096 45.9 -> 39.1, 220 x 3000 35.9 ->
+    // 37.7, 128 x 4096 31.2 -> 31.9) and keeps one unit per CU.  Lengths so
+    // unequal that this would take more than 3.5 slots per CU keep the other
+    // rules, so the partials fit the workspace a context starts with.
     int64_t equal_parts = 0;
     const int64_t n_cu = ctx->n_cu;
     if (total_rows > 0 && two_per_cu && ctx->opt_target_groups == 0 && 8 * (int64_t)n_seq >= 3 * n_cu &&
-        2 * n_cu > n_seq) {
+        2 * n_cu > n_seq && 16 * total_rows <= 9 * (int64_t)n_pos * n_seq) {
         const int64_t per = (total_rows + (2 * n_cu - n_seq) - 1) / (2 * n_cu - n_seq);
         const int64_t parts = (n_pos + per - 1) / per;
-        if (2 * parts * n_seq <= 7 * n_cu) equal_parts = parts;
+        if (2 * parts * n_seq <= 7 * n_cu && n_pos >= 768 * parts &&
+            (n_seq <= n_cu ? parts >= 3 : 8 * (int64_t)n_seq >= 9 * n_cu))
+            equal_parts = parts;
     }
     if (ctx->opt_split_len > 0) {
         len = (int)(((ctx->opt_split_len + round - 1) / round) * round);
