@@ -307,3 +307,28 @@ def test_any_shape_infinite_rows(ctx, nh, nkv, hd):
     for d in (dq, dk, dv, dki, dvi, do, dl, dout, dkn, dvn):
         d.free()
     assert ctx.check_device_error() == 0
+
+
+@pytest.mark.parametrize("nh,nkv,hd,cap", [(14, 2, 128, 1024), (14, 2, 128, 1025), (14, 2, 128, 4100), (12, 4, 96, 5000),
+                                           (40, 8, 128, 2000), (9, 3, 12, 4096), (5, 5, 256, 513), (9, 3, 66, 2100)])
+def test_layer_step_any_shape_large_capacity(ctx, nh, nkv, hd, cap):
+    """The layer step under a device-side position at capacities on both sides of the one from which it is split
+    (128 Ki floats of a kv head's rows), with 2 to 8 kv heads (the pairs of split and kv head are dealt to the
+    XCDs) and several head tiles, at positions on the edges of runs and at the capacity's end."""
+    kc, vc = oracle.normal(8300, (cap, nkv * hd)), oracle.normal(8301, (cap, nkv * hd))
+    dkc, dvc, dout = ctx.upload(kc), ctx.upload(vc), ctx.empty(nh * hd)
+    ctx.rope_prepare(hd, 1e6, cap)
+    for i, pos in enumerate((0, 1, 255, 256, 511, cap // 2, cap - 1)):
+        q, kn, vn = (oracle.normal(8310 + 3 * i + j, n * hd) for j, n in enumerate((nh, nkv, nkv)))
+        dq, dkn, dvn, dpos = ctx.upload(q), ctx.upload(kn), ctx.upload(vn), ctx.upload(np.array([pos], np.int32))
+        dout.fill_bytes(0xFF)
+        ctx.layer_attention_devpos(dq, dkn, dvn, dkc, dvc, dout, nh, nkv, hd, dpos, cap, 1e6)
+        ref, _, _ = oracle.layer_step(q, kn, vn, kc, vc, nh, nkv, hd, pos, 1e6)
+        assert_close(dout.numpy(), ref, f"layer {nh}/{nkv}/{hd} pos {pos} of {cap}")
+        for d in (dq, dkn, dvn, dpos):
+            d.free()
+    np.testing.assert_array_equal(dkc.numpy(), kc)
+    np.testing.assert_array_equal(dvc.numpy(), vc)
+    for d in (dkc, dvc, dout):
+        d.free()
+    assert ctx.check_device_error() == 0

@@ -1945,7 +1945,12 @@ __device__ __forceinline__ void any_body(const DecodeArgs& a) {
 // 4 bytes a lane (14 / 2 heads of 128 dims, 32 x 2048 rows: 142 us, 0.95 TB/s);
 // here a workgroup serves GT query heads of one kv head from one read of the
 // rows (32.6 us, 4.1 TB/s; one sequence of 4096 rows 147 -> 10.4 us).
-// grid = (split, kv head x head tile, sequence), NW waves.  Like the compiled
+// grid = (split, kv head x head tile, sequence), NW waves; a layer step in
+// several splits has grid (8 x head tile, (split, kv head) pairs / 8) instead,
+// which puts neighbouring pairs on different XCDs and the head tiles of a pair
+// on one: at a position far below the capacity the workgroups with rows are
+// spread over the chip, where (split, ...) left them all on one XCD (14 / 2
+// heads of 128 dims, capacity 32768, position 1000: 19.7 -> 10.2 us).  Like the compiled
 // group kernel with runtime head_dim: a row is served by LPR lanes of 8 dims
 // (16-byte chunks c and c + LPR of the head), a wave step covers 64 / LPR rows,
 // kAnyDepth steps of K and V are in flight, the online softmax keeps one
@@ -1988,7 +1993,15 @@ __device__ __forceinline__ void anyg_body(const DecodeArgs& a) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane % LPR, slot = lane / LPR;
-    const int split = blockIdx.x, kvh = blockIdx.y % n_kv, g0 = (blockIdx.y / n_kv) * GT, seq = blockIdx.z;
+    int split = blockIdx.x, kvh = blockIdx.y % n_kv, g0 = (blockIdx.y / n_kv) * GT;
+    const int seq = blockIdx.z;
+    if (MODE == kLayer && a.n_splits > 1) {
+        const int pair = blockIdx.y * 8 + (blockIdx.x & 7);
+        split = pair / n_kv;
+        kvh = pair - split * n_kv;
+        g0 = (blockIdx.x >> 3) * GT;
+        if (split >= a.n_splits) return;
+    }
     const int head0 = kvh * group + g0, n_g = min(GT, group - g0);  // this workgroup's query heads
     const size_t rowf = (size_t)n_kv * hd;
     int n_pos, pos;
@@ -2089,7 +2102,11 @@ __device__ __forceinline__ void anyg_body(const DecodeArgs& a) {
     };
     auto load_row8 = [&](Row& r, const float* head_row) {
         typedef float f32x4_t __attribute__((ext_vector_type(4)));
-        constexpr bool NT = GT > 1;  // one head per workgroup: other workgroups of the kv head read the row too
+        // Past the caches where the workgroup is mostly the row's only reader.  With one head per workgroup other
+        // workgroups read the row too; so they do with two in a layer step under a device-side position, whose order
+        // keeps the head tiles of a kv head on one XCD (64 / 8 heads of 128 dims, position 30000: 97 us past the
+        // caches, 58 through them; one tile of 8 heads, position 8900: 25.2 and 26.2).
+        constexpr bool NT = GT > (MODE == kLayer ? 2 : 1);
         const f32x4_t u = ld<NT, f32x4_t>(reinterpret_cast<const char*>(head_row + d0));
         const f32x4_t v = ld<NT, f32x4_t>(reinterpret_cast<const char*>(head_row + d1));
 #pragma unroll

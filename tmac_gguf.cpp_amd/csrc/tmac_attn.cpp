@@ -583,9 +583,26 @@ const float kQScale = (float)(1.4426950408889634 / 8.0);  // log2(e) / sqrt(64)
 // L2).  With one query head per kv head nothing is shared and the row kernel's
 // 8 waves are kept: as many splits as fit the CUs at one workgroup each, none
 // where the merge launch would buy no idle CU (5 / 5 heads of 256 dims, 32 x
-// 300 rows: 22.0 us in 320 units, 20.7 in 160; 64 x 256 29.0).  The partials fit the context's buffer, and the fixed scratch array of
-// the no-allocation entry point: fewer than 4 units of 8 heads per CU.
+// 300 rows: 22.0 us in 320 units, 16.9 in 160).  The partials fit the context's
+// buffer, and the fixed scratch array of the no-allocation entry point: fewer
+// than 4 units of 8 heads per CU.
+//
+// A layer step under a device-side position is launched for its capacity, and
+// most replays use little of it.  One head per workgroup (two or more from
+// kAnyPosUnits workgroups per split on), so that a short row range has n_head
+// workgroups and not n_kv_head.  No splits and no merge launch up to
+// kAnyPosWhole floats of a kv head's rows (1024 rows of 128 dims); beyond,
+// runs of at least kAnyPosRows rows, and no more than 4 workgroups per CU to
+// start for nothing.  us per captured step, 14 / 2 heads of 128 dims, at
+// positions 0 / 16 / 200 / 1000 / 4000 / 30000 of capacity 32768: the row
+// kernel 4.8 / 5.3 / 11.3 / 36.8 / 145 / 1056, splits as for a position known
+// at launch 9.1 / 10.9 / 16.5 / 16.7 / 19.1 / 39.7, now 5.5 / 5.5 / 6.4 / 9.1 /
+// 9.9 / 28.9; of capacity 256, positions 16 / 200: 5.3 / 11.3, 5.3 / 7.2, 3.6 /
+// 4.8; of capacity 1024, position 1000: 36.8, 7.5, 10.4.  The merge launch of
+// the larger capacities costs the positions below about 20 up to 1.2 us over
+// the row kernel.
 constexpr int kAnyTargetPerCu = 2, kAnyMinRows = 128;
+constexpr int kAnyPosWhole = 128 * 1024, kAnyPosRows = 256, kAnyPosUnits = 32;
 int run_decode_any(tmac_context* ctx, hipStream_t stream, const Kernels& k, DecodeArgs& a, int n_seq, int grid_rows,
                    int n_kv_head) {
     a.n_kv_head = n_kv_head;
@@ -598,9 +615,18 @@ int run_decode_any(tmac_context* ctx, hipStream_t stream, const Kernels& k, Deco
     auto tiles = [&] { return (group + (1 << gt) - 1) >> gt; };
     if (a.head_dim % 4 != 0 || (int64_t)n_kv_head * group > 65535)
         return launch(ctx, k.any, (unsigned)a.n_head, (unsigned)n_seq, tmac::kAnyWavesHost * 64, stream, &a);
+    const bool by_pos = a.pos_dev != nullptr;
     const int64_t units = (int64_t)n_seq * n_kv_head * tiles();
     int64_t want = group == 1 ? ctx->n_cu / units : (kAnyTargetPerCu * (int64_t)ctx->n_cu + units - 1) / units;
     want = std::min<int64_t>(want, std::min(grid_rows / kAnyMinRows, kMaxSplits));
+    if (by_pos) {
+        const bool whole = (int64_t)grid_rows * std::max(a.head_dim, kHeadDim) <= kAnyPosWhole;
+        const int most = gt;
+        gt = 0;
+        while (!whole && gt < most && n_kv_head * tiles() > kAnyPosUnits) gt++;
+        want = std::min(std::min(grid_rows / kAnyPosRows, 4 * ctx->n_cu / (n_kv_head * tiles())), kMaxSplits);
+        if (whole) want = 1;
+    }
     if (want > 1) {
         const int64_t len = (((int64_t)grid_rows + want - 1) / want + 31) / 32 * 32;
         const int n_splits = (int)((grid_rows + len - 1) / len);
@@ -613,8 +639,13 @@ int run_decode_any(tmac_context* ctx, hipStream_t stream, const Kernels& k, Deco
     }
     while (gt > 0 && (int64_t)n_seq * n_kv_head * tiles() * a.n_splits * 2 <= ctx->n_cu) gt--;
     const int n4 = a.head_dim / 4, li = n4 <= 8 ? 0 : n4 <= 16 ? 1 : n4 <= 32 ? 2 : 3;  // 4 << li lanes of 8 dims
-    int rc = launch(ctx, ctx->any_group[k.any_mode][li][gt], (unsigned)a.n_splits, (unsigned)(n_kv_head * tiles()),
-                    tmac::any_group_waves(1 << gt) * 64, stream, &a, (unsigned)n_seq);
+    unsigned gx = (unsigned)a.n_splits, gy = (unsigned)(n_kv_head * tiles());
+    if (k.any_mode == kModeLayer && a.n_splits > 1) {  // (the kernel's order of a split layer step)
+        gx = 8 * (unsigned)tiles();
+        gy = (unsigned)(n_kv_head * a.n_splits + 7) / 8;
+    }
+    int rc = launch(ctx, ctx->any_group[k.any_mode][li][gt], gx, gy, tmac::any_group_waves(1 << gt) * 64, stream, &a,
+                    (unsigned)n_seq);
     if (rc || a.n_splits == 1) return rc;
     return launch(ctx, ctx->any_combine[k.any_mode], (unsigned)a.n_head, (unsigned)n_seq, kAnyMaxDim, stream, &a);
 }
