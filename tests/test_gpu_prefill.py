@@ -431,3 +431,23 @@ def test_prefill_infinity_in_v(ctx, n_q, prefix):
         got = run(ctx, q, k, vi, 1, n_q, prefix, cap, n_head, n_kv).reshape(n_q, -1)
         assert np.all(got[:, first] == np.inf), f"row {row}"
         assert_close(got[:, ~first], ref.reshape(n_q, -1)[:, ~first], f"row {row}, the other dims")
+
+
+@pytest.mark.parametrize("n_seq,n_q,prefix,n_head,n_kv", [
+    (3, 140, 0, 14, 2),   # 9 blocks: a band of 8 and one more, 6 pairs
+    (5, 250, 20, 14, 2),  # 16 blocks, two bands, 10 pairs
+    (7, 100, 0, 14, 2),   # 7 blocks, no whole band, 14 pairs
+    (3, 180, 7, 1, 1),    # 3 pairs
+    (1, 129, 100, 16, 4), (11, 33, 5, 8, 1)])
+def test_prefill_block_order(ctx, n_seq, n_q, prefix, n_head, n_kv):
+    """Every (query block, kv head, sequence) is computed once whatever the number of pairs and
+    blocks that the order deals to the XCDs: against the oracle, into a NaN-filled output."""
+    cap = prefix + n_q
+    q, k, v = (bf16_round(a) for a in make(970 + n_q, n_seq, n_q, prefix, cap, n_head, n_kv))
+    dq, dk, dv, dout = ctx.upload(q), ctx.upload(k), ctx.upload(v), ctx.empty(q.shape)
+    dout.fill_bytes(0xFF)
+    ctx.prefill(dq, dk, dv, dout, n_seq, n_q, prefix, cap, n_head, n_kv, HD)
+    ref = oracle.prefill(q, k, v, n_seq, n_q, prefix, cap, n_head, n_kv, HD, n_threads=8)
+    assert_close(dout.numpy().ravel(), ref.ravel(), f"{n_seq}x{n_q} prefix {prefix} heads {n_head}/{n_kv}")
+    for d in (dq, dk, dv, dout):
+        d.free()

@@ -2376,12 +2376,8 @@ TMAC_DECODE_KERNELS(8, 1)
 //
 // Attention workgroup = (16-query block, kv head, sequence), or a run of its
 // keys, 8 waves.  The 1-D grid holds the blocks from the last (most keys) to
-// the first, the (sequence, kv head) pairs of a block side by side: workgroups
-// are dealt to the 8 XCDs round-robin, so every XCD gets an even mix of long
-// and short blocks, longest first, and with 1, 2, 4 or a multiple of 8 pairs
-// an XCD reads only its own share of the tiles.  (An order that gave each XCD
-// a contiguous run of blocks left the XCDs with the last blocks of a prompt
-// working alone: one prompt of 2999 rows 80.5 us, 49.2 in this order.)
+// the first, so that every XCD (workgroups are dealt to them round-robin) gets
+// an even mix of long and short blocks, longest first (prefill_block).
 // Where the blocks are fewer than the CUs, each block's keys are cut into runs
 // of `split` stages, one workgroup each, and a second launch merges the
 // partials (prefill_plan in tmac_attn.cpp).  Wave w computes tiles 2 * (w / 4) and 2 * (w / 4) + 1 of every stage
@@ -2577,6 +2573,32 @@ __device__ __forceinline__ bool prefill_unit(const PrefillArgs& a, int rank, int
     return false;
 }
 
+// Whole blocks: workgroup id -> (sequence, kv head) pair and block.  Bands of 8
+// blocks of every pair, from the last blocks down: an XCD takes the n_sk units
+// of a band that lie next to each other pair by pair, so it reads the tiles of
+// n_sk / 8 + 1 pairs or so whatever their number, and the bands alternate
+// between longest and shortest block first.  us, an XCD with a contiguous run
+// of all blocks / pairs of a block dealt out in turn / this order: one prompt
+// of 2999 rows 80.0 / 53.1 / 52.7, 3 x 512 queries after 1536 rows 36.2 / 37.6
+// / 36.4, 6 x 512 65.2 / 66.5 / 64.5, 3 x 1000 after none 32.9 / 28.6 / 28.1,
+// 11 x 200 after 300 27.2 / 28.3 / 26.4.
+__device__ __forceinline__ void prefill_block(const PrefillArgs& a, int id, int& sk, int& qblk) {
+    const int band = 8 * a.n_sk, full = a.n_qblk >> 3;  // whole bands
+    const int x = id & 7;
+    int rank;
+    if (id < full * band) {
+        const int i = id >> 3, b = i / a.n_sk, t = x * a.n_sk + (i - b * a.n_sk);
+        sk = t >> 3;
+        rank = 8 * b + ((b & 1) ? 7 - (t & 7) : t & 7);
+    } else {  // the last band, of fewer blocks
+        const int rem = a.n_qblk & 7, n = rem * a.n_sk, i = (id - full * band) >> 3;
+        const int t = x * (n >> 3) + min(x, n & 7) + i;
+        sk = t / rem;
+        rank = 8 * full + (t - sk * rem);
+    }
+    qblk = a.n_qblk - 1 - rank;
+}
+
 // RUNS: units are key runs of the blocks (a.split > 0); otherwise whole blocks,
 // in a kernel without the run code (4 x 512 queries on 1536 rows: 37.4 us with
 // it, 37.0 without).
@@ -2590,9 +2612,13 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int pair = wave & 3, part = wave >> 2;  // head pair, half of the stage (two tiles)
 
-    const int sk = blockIdx.x % a.n_sk;  // (sequence, kv head)
-    int qblk = a.n_qblk - 1 - (int)(blockIdx.x / a.n_sk), part_idx = 0, n_act = 1;
-    if (RUNS && !prefill_unit(a, blockIdx.x / a.n_sk, qblk, part_idx, n_act)) return;
+    int sk, qblk, part_idx = 0, n_act = 1;  // sk: (sequence, kv head)
+    if (RUNS) {
+        sk = blockIdx.x % a.n_sk;
+        if (!prefill_unit(a, blockIdx.x / a.n_sk, qblk, part_idx, n_act)) return;
+    } else {
+        prefill_block(a, blockIdx.x, sk, qblk);
+    }
     const int seq = sk / KV, kv = sk - seq * KV;
     const int q0 = qblk * QB;
     const int q_last = min(q0 + QB, a.n_q) - 1;
