@@ -2929,10 +2929,11 @@ __device__ __forceinline__ void prefill_combine_body(const PrefillArgs& a) {
 #pragma unroll
         for (int j = 0; j < kMergeRuns; ++j) {
             const float w = (m[j] == kNegInf) ? 0.f : fast_exp2(m[j] - nm);
-            const bool in = u0 + j < n_act;  // (repeats of the last run stay out: 0 * inf is NaN)
-            L = in ? fmaf(l[j], w, L) : L;
+            if (u0 + j < n_act) {  // (repeats of the last run stay out: 0 * inf is NaN)
+                L = fmaf(l[j], w, L);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) A[i] = in ? fmaf(x[j][i], w, A[i]) : A[i];
+                for (int i = 0; i < 4; ++i) A[i] = fmaf(x[j][i], w, A[i]);
+            }
         }
         M = nm;
     }
