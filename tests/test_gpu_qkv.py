@@ -280,3 +280,26 @@ def test_gemv_rows_and_rounds(ctx, qtype, rows, cols):
     np.testing.assert_array_equal(dy.numpy(), got + got)
     for d in (dw, dx, dy):
         d.free()
+
+
+@pytest.mark.parametrize("qtype,rows", [(oracle.Q6_K, 2047), (oracle.Q6_K, 2049), (oracle.Q4_K, 16385),
+                                        (oracle.Q5_0, 16385), (oracle.Q8_0, 16385)])
+@pytest.mark.parametrize("cols", [256, 2304])
+def test_gemv_rows_keep_their_bits_in_a_large_matrix(ctx, qtype, rows, cols):
+    """A row's sum has the same bits whatever the number of rows chooses (rows per wave, super-blocks in
+    flight; 256 CUs: Q6_K changes at 2,048 rows, the others at 16,384): rows of the whole matrix against
+    calls on 64 rows of it, at its start and its end."""
+    rng = np.random.default_rng(rows + cols)
+    raw = rng.integers(0, 256, (rows * (cols // (256 if qtype >= tmac_attn.TMAC_Q4_K else 32)),
+                                oracle.BLOCK_BYTES[qtype]), dtype=np.uint8)
+    for at in ([208] if qtype == oracle.Q6_K else [0, 2] if qtype == oracle.Q4_K else [0]):
+        raw[:, at:at + 2] = rng.uniform(1e-4, 2e-4, (raw.shape[0], 1)).astype(np.float16).view(np.uint8)
+    dw, dx = ctx.upload(raw.reshape(-1)), ctx.upload(rng.standard_normal(cols).astype(np.float32))
+    dy, dpart = ctx.empty(rows), ctx.empty(64)
+    ctx.matmul(qtype, rows, cols, dw, dx, dy)
+    whole = dy.numpy().view(np.uint32)
+    for r0 in (0, rows - 65, rows - 64):
+        ctx.matmul(qtype, 64, cols, dw.ptr + r0 * (raw.size // rows), dx, dpart)
+        np.testing.assert_array_equal(dpart.numpy().view(np.uint32), whole[r0:r0 + 64], err_msg=f"rows from {r0}")
+    for d in (dw, dx, dy, dpart):
+        d.free()

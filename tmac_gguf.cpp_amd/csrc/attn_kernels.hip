@@ -4026,7 +4026,8 @@ extern "C" __global__ __launch_bounds__(256) void tmac_copy(CopyArgs a) {
 // expression (Q6_K: d * scale * q, exact; Q4_K: d * sc * q - dmin * m, exact
 // products and one rounding); the row sum is one FMA per element and a wave
 // reduction.  Latency-bound where the rows are few: the loads of 8 super-blocks
-// are in flight together (896 x 4864: Q4_K 8.2 -> 4.1 us, Q6_K 6.1 -> 4.3).
+// are in flight together (896 x 4864: Q4_K 8.2 -> 4.1 us, Q6_K 6.1 -> 4.3);
+// with more rows than that needs, fewer (matmul_common in tmac_attn.cpp).
 // This lane's 4 weights of a super-block as loaded, and dequantised.
 template <bool Q6>
 struct KBlock;
@@ -4082,9 +4083,8 @@ struct KBlock<false> {
 };
 
 // RW rows per wave; the loads of kSbRound super-blocks are in flight together.
-template <bool Q6, int RW>
+template <bool Q6, int RW, int kSbRound>
 __device__ __forceinline__ void kq_body(const KqArgs& a) {
-    constexpr int kSbRound = RW == 1 ? 8 : 2;
     const int lane = threadIdx.x & 63;
     const int r0 = (blockIdx.x * kQkvWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * RW;
     if (r0 >= a.rows) return;
@@ -4119,7 +4119,8 @@ __device__ __forceinline__ void kq_body(const KqArgs& a) {
             }
     };
     int sb = 0;
-    for (; sb + kSbRound <= nsb; sb += kSbRound) round(sb, IntTag<kSbRound>{});
+    if constexpr (kSbRound > 1)
+        for (; sb + kSbRound <= nsb; sb += kSbRound) round(sb, IntTag<kSbRound>{});
     for (; sb < nsb; ++sb) round(sb, IntTag<1>{});
 #pragma unroll
     for (int j = 0; j < RW; ++j) {
@@ -4127,9 +4128,12 @@ __device__ __forceinline__ void kq_body(const KqArgs& a) {
         if (lane == 0 && j < n_rows) a.y[r0 + j] = a.bias ? v + a.bias[r0 + j] : v;
     }
 }
-extern "C" __global__ __launch_bounds__(kQkvWaves * 64) void tmac_matmul_q6_k(KqArgs a) { kq_body<true, 1>(a); }
-extern "C" __global__ __launch_bounds__(kQkvWaves * 64) void tmac_matmul_q4_k(KqArgs a) { kq_body<false, 1>(a); }
-extern "C" __global__ __launch_bounds__(kQkvWaves * 64) void tmac_gemv_rows_q4_k(KqArgs a) { kq_body<false, kGemvRows>(a); }
+extern "C" __global__ __launch_bounds__(kQkvWaves * 64) void tmac_matmul_q6_k(KqArgs a) { kq_body<true, 1, 8>(a); }
+extern "C" __global__ __launch_bounds__(kQkvWaves * 64) void tmac_matmul_q4_k(KqArgs a) { kq_body<false, 1, 8>(a); }
+extern "C" __global__ __launch_bounds__(kQkvWaves * 64) void tmac_gemv_rows_q4_k(KqArgs a) {
+    kq_body<false, kGemvRows, 2>(a);
+}
+extern "C" __global__ __launch_bounds__(kQkvWaves * 64) void tmac_gemv_rows_q6_k(KqArgs a) { kq_body<true, 1, 1>(a); }
 
 // Fills a 16-bit cache from fp32 values, rounding to nearest even.
 extern "C" __global__ __launch_bounds__(256) void tmac_cvt16(CvtArgs a) {

@@ -133,7 +133,7 @@ struct tmac_context {
     hipFunction_t any_combine[3] = {};
     hipFunction_t k_rope = nullptr, k_copy = nullptr, k_pos = nullptr, k_qkv = nullptr, k_cvt16 = nullptr,
                   k_cvt_q8 = nullptr;
-    // quantized GEMV of a large matrix; K-quants: [Q6_K][large matrix] (Q6_K: one kernel for both)
+    // quantized GEMV of a large matrix; K-quants: [Q6_K][large matrix]
     hipFunction_t k_gemv_q8 = nullptr, k_gemv_q5 = nullptr, k_kq[2][2] = {};
     float* ws = nullptr;
     size_t ws_floats = 0;
@@ -1012,6 +1012,7 @@ int tmac_init(tmac_context** out, int device) {
         (e = get_function(ctx, &ctx->k_kq[0][0], "tmac_matmul_q4_k")) != hipSuccess ||
         (e = get_function(ctx, &ctx->k_kq[0][1], "tmac_gemv_rows_q4_k")) != hipSuccess ||
         (e = get_function(ctx, &ctx->k_kq[1][0], "tmac_matmul_q6_k")) != hipSuccess ||
+        (e = get_function(ctx, &ctx->k_kq[1][1], "tmac_gemv_rows_q6_k")) != hipSuccess ||
         (e = get_function(ctx, &ctx->k_cvt_q8, "tmac_cvt_q8")) != hipSuccess)
         return bail(hip_fail(ctx, e, "hipModuleGetFunction"));
     if ((e = hipStreamCreateWithFlags(&ctx->aux, hipStreamNonBlocking)) != hipSuccess)
@@ -1680,8 +1681,13 @@ int tmac_elem_op(tmac_context* ctx, tmac_stream stream, int op, float* data, con
 
 // GEMV grids: one output row per wave, or kGemvRows in a large matrix, whose
 // rows still give every SIMD several waves (Q8_0, 4 rows a wave against 1, us:
-// 32000 x 1024 14.8 -> 10.0, 16000 x 1024 equal).  Q6_K stays at one row: its
-// loads are 4 bytes a lane whatever the rows (32000 x 4864 73 us, 84 with 4).
+// 32000 x 1024 14.8 -> 10.0, 16000 x 1024 equal; Q5_0 32000 x 1024 15.2 ->
+// 10.5, Q4_K 14.3 -> 11.1).  Q6_K stays at one row: its loads are 4 bytes a lane
+// whatever the rows (32000 x 4864 73 us, 84 with 4).  From 8 rows per CU on its
+// waves hide the loads themselves and take the super-blocks one by one: eight
+// in flight at once are faster below (896 x 4864 5.1 us, 6.0 one by one; 2048 x
+// 4864 6.7 both) and slower above (8192 x 2048 9.1 and 7.9, 32000 x 4864 55.3
+// and 51.4, 151936 x 2048 120 and 96).
 static bool large_gemv(const tmac_context* ctx, int rows) { return rows >= 64 * ctx->n_cu; }
 static unsigned gemv_grid(int64_t rows, bool large) {
     const int per = kQkvWaves * (large ? tmac::kGemvRows : 1);
@@ -1747,8 +1753,8 @@ static int matmul_common(tmac_context* ctx, hipStream_t stream, int qtype, int r
         if (rows == 0) return TMAC_OK;
         if ((rc = set_device(ctx))) return rc;
         KqArgs a{(const uint8_t*)w, x, accumulate ? y : nullptr, y, rows, cols, qtype};
-        const bool large = qtype == TMAC_Q4_K && large_gemv(ctx, rows);
-        return launch(ctx, ctx->k_kq[qtype == TMAC_Q6_K][large], gemv_grid(rows, large), 1, kQkvWaves * 64, stream, &a);
+        const bool q6 = qtype == TMAC_Q6_K, large = q6 ? rows >= 8 * ctx->n_cu : large_gemv(ctx, rows);
+        return launch(ctx, ctx->k_kq[q6][large], gemv_grid(rows, large && !q6), 1, kQkvWaves * 64, stream, &a);
     }
     return qkv_common(ctx, stream, nullptr, nullptr, w, x, nullptr, nullptr, accumulate ? y : nullptr, nullptr,
                       nullptr, y, 0, 0, rows, cols, qtype == TMAC_Q8_0);
