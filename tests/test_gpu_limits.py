@@ -259,3 +259,15 @@ def test_length_bound_is_exact(ctx, dt, entry):
         ctx.set_option(tmac_attn.TMAC_OPT_STREAM_K, 1)
     for d in (dq, dout, dk, dv, doff, dlen, dtab, dpos, dkn, dvn):
         d.free()
+
+
+def test_init_leaves_no_runtime_error(ctx):
+    """tmac_init looks each kernel up in several code objects; the misses leave no error behind that
+    the next user of the HIP runtime in the thread would report as its own."""
+    with open("/proc/self/maps") as f:
+        path = next(line.split()[-1] for line in f if "libamdhip64" in line)
+    hip = ctypes.CDLL(path)
+    hip.hipGetLastError()
+    with tmac_attn.Context(0):
+        assert hip.hipPeekAtLastError() == 0
+    assert hip.hipGetLastError() == 0

@@ -217,12 +217,15 @@ int set_device(tmac_context* ctx) {
     return TMAC_OK;
 }
 
-// Looks a kernel up in whichever code object part holds it.
+// Looks a kernel up in whichever code object part holds it.  The parts that do
+// not hold it leave the runtime's last error set, which the caller's next
+// library would report as its own: it is cleared.
 hipError_t get_function(tmac_context* ctx, hipFunction_t* f, const char* name) {
-    for (auto m : ctx->modules)
-        if (m && hipModuleGetFunction(f, m, name) == hipSuccess) return hipSuccess;
+    hipError_t found = hipErrorNotFound;
+    for (int i = 0; i < kCodeParts && found != hipSuccess; i++)
+        if (ctx->modules[i] && hipModuleGetFunction(f, ctx->modules[i], name) == hipSuccess) found = hipSuccess;
     (void)hipGetLastError();
-    return hipErrorNotFound;
+    return found;
 }
 
 bool capturing(hipStream_t s) {
