@@ -2906,11 +2906,12 @@ __device__ __forceinline__ void prefill_combine_body(const PrefillArgs& a) {
     if (n_act <= 1) return;
     const float* p0 = a.part + (((size_t)sk * a.n_qblk + qblk) * a.n_parts * G + g) * kPrefillPartFloats + lane;
     float M = kNegInf, L = 0.f, A[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int u0 = 0; u0 < n_act; u0 += kMergeRuns) {
+    auto merge = [&](int u0, auto whole) {  // kMergeRuns runs, or the last n_act - u0
+        constexpr bool WHOLE = decltype(whole)::value;
         float m[kMergeRuns], l[kMergeRuns], x[kMergeRuns][4];
 #pragma unroll
         for (int j = 0; j < kMergeRuns; ++j) {
-            const float* p = p0 + (size_t)min(u0 + j, n_act - 1) * G * kPrefillPartFloats;
+            const float* p = p0 + (size_t)(WHOLE ? u0 + j : min(u0 + j, n_act - 1)) * G * kPrefillPartFloats;
             m[j] = p[16 * 64];
             l[j] = p[17 * 64];
 #pragma unroll
@@ -2918,9 +2919,7 @@ __device__ __forceinline__ void prefill_combine_body(const PrefillArgs& a) {
         }
         float nm = M;
 #pragma unroll
-        for (int j = 0; j < kMergeRuns; ++j) {
-            nm = fmaxf(nm, m[j]);
-        }
+        for (int j = 0; j < kMergeRuns; ++j) nm = fmaxf(nm, m[j]);
         // (nm is finite: every column sees key 0, which is in the first run)
         const float sc = (M == kNegInf) ? 0.f : fast_exp2(M - nm);
         L *= sc;
@@ -2929,14 +2928,16 @@ __device__ __forceinline__ void prefill_combine_body(const PrefillArgs& a) {
 #pragma unroll
         for (int j = 0; j < kMergeRuns; ++j) {
             const float w = (m[j] == kNegInf) ? 0.f : fast_exp2(m[j] - nm);
-            if (u0 + j < n_act) {  // (repeats of the last run stay out: 0 * inf is NaN)
-                L = fmaf(l[j], w, L);
+            const bool in = WHOLE || u0 + j < n_act;  // (repeats of the last run stay out: 0 * inf is NaN)
+            L = in ? fmaf(l[j], w, L) : L;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) A[i] = fmaf(x[j][i], w, A[i]);
-            }
+            for (int i = 0; i < 4; ++i) A[i] = in ? fmaf(x[j][i], w, A[i]) : A[i];
         }
         M = nm;
-    }
+    };
+    int u0 = 0;
+    for (; u0 + kMergeRuns <= n_act; u0 += kMergeRuns) merge(u0, BoolTag<true>{});
+    if (u0 < n_act) merge(u0, BoolTag<false>{});
     const int qi = qblk * kPrefillQueries + (lane & 15);
     if (qi >= a.n_q) return;
     const int seq = sk / KV, kv = sk - seq * KV;
