@@ -172,7 +172,7 @@ constexpr int kQkvWaves = 4;         // waves per workgroup, one output row each
 constexpr int kGemvRows = 4;
 
 // y = W x (+ bias) for K-quant weights: rows of cols / 256 super-blocks, Q4_K
-// (type 12, 144 bytes) or Q6_K (type 14, 210 bytes).  bias may equal y (the
+// (144 bytes) or Q6_K (210 bytes), a kernel each.  bias may equal y (the
 // residual form y += W x).
 struct KqArgs {
     const uint8_t* w;
@@ -181,7 +181,6 @@ struct KqArgs {
     float* y;
     int rows;
     int cols;
-    int type;
 };
 
 struct PosArgs {

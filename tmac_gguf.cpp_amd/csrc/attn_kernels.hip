@@ -2550,8 +2550,8 @@ __device__ __forceinline__ int prefill_stages(const PrefillArgs& a, int b) {
 // Unit `rank` of a (sequence, kv head), blocks from the last (most keys) to
 // the first: its query block, which run of `split` stages of the block's keys
 // it attends and how many runs the block has.  Every wave computes the same
-// answer (lane l takes block l of a round of 64; blocks number a few per CU
-// where keys are split).
+// answer (lane l takes block l of a round of 64; keys are split only where the
+// blocks of all pairs are at most half the CUs).
 __device__ __forceinline__ bool prefill_unit(const PrefillArgs& a, int rank, int& qblk, int& part, int& n_act) {
     const int lane = threadIdx.x & 63;
     int base = 0;

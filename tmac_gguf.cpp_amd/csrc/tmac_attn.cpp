@@ -1774,7 +1774,7 @@ static int matmul_common(tmac_context* ctx, hipStream_t stream, int qtype, int r
             return fail(ctx, TMAC_ERR_MISALIGNED, "matmul: x 16-byte, weights 2-byte, y 4-byte aligned");
         if (rows == 0) return TMAC_OK;
         if ((rc = set_device(ctx))) return rc;
-        KqArgs a{(const uint8_t*)w, x, accumulate ? y : nullptr, y, rows, cols, qtype};
+        KqArgs a{(const uint8_t*)w, x, accumulate ? y : nullptr, y, rows, cols};
         const bool q6 = qtype == TMAC_Q6_K, large = q6 ? rows >= 8 * ctx->n_cu : large_gemv(ctx, rows);
         return launch(ctx, ctx->k_kq[q6][large], gemv_grid(rows, large && !q6), 1, kQkvWaves * 64, stream, &a);
     }
