@@ -144,8 +144,7 @@ struct tmac_context {
     float* part = nullptr;
     size_t part_floats = 0;
     int* err = nullptr;
-    // The stream of the library's own copies and fills, once
-    // tmac_check_device_error has made it (AuxStream).
+    // The stream tmac_check_device_error reads the error word on (AuxStream).
     hipStream_t aux = nullptr;
     // RoPE row caches of the device-side position counters the layer entry
     // points have seen (kPosSlotBlocks blocks of kPosSlotBytes, allocated and
@@ -250,17 +249,18 @@ bool quiesce(tmac_context* ctx) {
 // The library's own copies and fills (tables, tags, the error word) go on a
 // non-blocking stream and wait for it alone: on this runtime a legacy-stream
 // copy or a device-wide synchronize issued while a stream of another thread is
-// capturing fails and ends that capture.  The stream is made for each, unless
-// the context holds one (tmac_check_device_error keeps it: 20 us a call, 64
-// with a stream of its own): a held stream takes one of the process's few
-// hardware queues, and a program's own stream then came to lie on the third,
-// where the same kernels took longer (captured 24-layer attention block 241 us,
-// 238 on the second; layer step of 64 paged sequences 96.6 and 94.3).
+// capturing fails and ends that capture.  The stream is made for each: a stream
+// that has been used takes one of the process's few hardware queues, and a
+// program's own stream then came to lie on the third, where the same kernels
+// took longer (captured 24-layer attention block 241 us, 238 on the second;
+// layer step of 64 paged sequences 96.6 and 94.3).  Only the error check, which
+// may be called often, uses the one the context holds (`held`; 20 us a call, 64
+// with a stream made for it).
 struct AuxStream {
     hipStream_t s, own = nullptr;
     hipError_t e = hipSuccess;
-    explicit AuxStream(const tmac_context* ctx) : s(ctx->aux) {
-        if (s) return;
+    AuxStream(const tmac_context* ctx, bool held) : s(ctx->aux) {
+        if (held) return;
         e = hipStreamCreateWithFlags(&own, hipStreamNonBlocking);
         s = own;
     }
@@ -271,14 +271,15 @@ struct AuxStream {
     AuxStream& operator=(const AuxStream&) = delete;
 };
 
-hipError_t aux_fill(const tmac_context* ctx, void* p, int value, size_t bytes) {
-    AuxStream aux(ctx);
+hipError_t aux_fill(const tmac_context* ctx, void* p, int value, size_t bytes, bool held = false) {
+    AuxStream aux(ctx, held);
     if (aux.e == hipSuccess) aux.e = hipMemsetAsync(p, value, bytes, aux.s);
     return aux.e != hipSuccess ? aux.e : hipStreamSynchronize(aux.s);
 }
 
-hipError_t aux_copy(const tmac_context* ctx, void* dst, const void* src, size_t bytes, hipMemcpyKind kind) {
-    AuxStream aux(ctx);
+hipError_t aux_copy(const tmac_context* ctx, void* dst, const void* src, size_t bytes, hipMemcpyKind kind,
+                    bool held = false) {
+    AuxStream aux(ctx, held);
     if (aux.e == hipSuccess) aux.e = hipMemcpyAsync(dst, src, bytes, kind, aux.s);
     return aux.e != hipSuccess ? aux.e : hipStreamSynchronize(aux.s);
 }
@@ -869,6 +870,7 @@ int tmac_init(tmac_context** out, int device) {
         if (ctx->part) (void)hipFree(ctx->part);
         if (ctx->err) (void)hipFree(ctx->err);
         if (ctx->pos_slot_pool) (void)hipFree(ctx->pos_slot_pool);
+        if (ctx->aux) (void)hipStreamDestroy(ctx->aux);
         for (auto& m : ctx->modules)
             if (m) (void)hipModuleUnload(m);
         delete ctx;
@@ -1040,6 +1042,8 @@ int tmac_init(tmac_context** out, int device) {
         (e = get_function(ctx, &ctx->k_kq[1][1], "tmac_gemv_rows_q6_k")) != hipSuccess ||
         (e = get_function(ctx, &ctx->k_cvt_q8, "tmac_cvt_q8")) != hipSuccess)
         return bail(hip_fail(ctx, e, "hipModuleGetFunction"));
+    if ((e = hipStreamCreateWithFlags(&ctx->aux, hipStreamNonBlocking)) != hipSuccess)
+        return bail(hip_fail(ctx, e, "hipStreamCreateWithFlags"));
     if ((e = hipMalloc(&ctx->err, sizeof(int))) != hipSuccess) return bail(hip_fail(ctx, e, "hipMalloc"));
     if ((e = aux_fill(ctx, ctx->err, 0, sizeof(int))) != hipSuccess) return bail(hip_fail(ctx, e, "hipMemsetAsync"));
     if ((e = hipMalloc(&ctx->pos_slot_pool, (size_t)tmac::kPosSlotBlocks * tmac::kPosSlotBytes)) != hipSuccess)
@@ -1878,11 +1882,10 @@ int tmac_check_device_error(tmac_context* ctx) {
     if (rc) return rc;
     if ((rc = set_device(ctx))) return rc;
     (void)quiesce(ctx);
-    if (!ctx->aux) HIP_TRY(ctx, hipStreamCreateWithFlags(&ctx->aux, hipStreamNonBlocking));
     int v = 0;
-    HIP_TRY(ctx, aux_copy(ctx, &v, ctx->err, sizeof(int), hipMemcpyDeviceToHost));
+    HIP_TRY(ctx, aux_copy(ctx, &v, ctx->err, sizeof(int), hipMemcpyDeviceToHost, true));
     if (v) {
-        HIP_TRY(ctx, aux_fill(ctx, ctx->err, 0, sizeof(int)));
+        HIP_TRY(ctx, aux_fill(ctx, ctx->err, 0, sizeof(int), true));
         return fail(ctx, TMAC_ERR_DEVICE_FAULT, "a kernel saw a device-side position outside its table or cache");
     }
     return TMAC_OK;
